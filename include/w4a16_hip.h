@@ -148,6 +148,18 @@ int w4a16_dequantize_f16(const uint8_t* packed_weights, const void* scales,
                          void* stream);
 
 /*
+ * Quantize weights [N, K] (fp16: weight_bytes 2, fp32: 4; row-major) to packed
+ * codes uint8 [N, K/2] and fp16 scales [N, K/G]: per group s = amax|w| / 7 in
+ * fp32 (1.0 for a zero group), codes clamp(round_half_even(w / s), -7, 7),
+ * stored scale fp16(s). Same bytes as reference w4a16/quantization.py:65-113,
+ * which has no native form. group_size a power of two from 16 to 512, K a
+ * multiple of it, weights 16-byte, packed_weights 4-byte aligned.
+ */
+int w4a16_quantize_pack(const void* weights, int weight_bytes,
+                        uint8_t* packed_weights, void* scales, int64_t N,
+                        int64_t K, int64_t group_size, void* stream);
+
+/*
  * Shape validator shared by the torch op and host-only tests. Arguments are
  * the sizes the three tensors carry. Returns W4A16_OK or an error code whose
  * w4a16_last_error() text matches the reference's TORCH_CHECK messages

@@ -68,6 +68,7 @@ SIGNATURES = {
         ctypes.c_int,
         [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp] + [ctypes.c_int] * 5 + [_vp, _i64],
     ),
+    "w4a16_quantize_pack": (ctypes.c_int, [_vp, ctypes.c_int, _vp, _vp, _i64, _i64, _i64, _vp]),
     "w4a16_last_error": (ctypes.c_char_p, []),
     "w4a16_version": (ctypes.c_char_p, []),
 }

@@ -1,6 +1,6 @@
 // Thin libtorch shim over the W4A16 C ABI: registers the torch ops
 // w4a16::linear and w4a16::dequantize with the schemas of reference
-// csrc/int4_linear.cpp:16-23, implemented on the CUDA dispatch key (which is
+// csrc/int4_linear.cpp:16-23 and w4a16::quantize (the reference quantizes in torch ops), implemented on the CUDA dispatch key (which is
 // the HIP device on PyTorch-ROCm), and exposes an empty Python module so that
 // importing the extension registers the ops (reference csrc/int4_linear.cpp:30).
 //
@@ -92,16 +92,37 @@ at::Tensor dequantize(const at::Tensor& packed_weights, const at::Tensor& scales
     return weights;
 }
 
+// Weights [N, K] -> (packed uint8 [N, K / 2], scales fp16 [N, K / G]); the
+// caller (nibble_amd/quantization.py) has made the quantizer's own checks.
+std::tuple<at::Tensor, at::Tensor> quantize(const at::Tensor& weights, int64_t group_size) {
+    TORCH_CHECK(weights.is_cuda(), "weights must be a CUDA tensor");
+    TORCH_CHECK(weights.scalar_type() == at::kHalf || weights.scalar_type() == at::kFloat,
+                "weights must have dtype torch.float16 or torch.float32");
+    TORCH_CHECK(weights.dim() == 2 && weights.is_contiguous(), "weights must be contiguous with shape [N, K]");
+    TORCH_CHECK(group_size > 0 && weights.size(1) % group_size == 0, "K must be divisible by group_size");
+    const int64_t N = weights.size(0);
+    const int64_t K = weights.size(1);
+    const c10::DeviceGuard guard(weights.device());
+    at::Tensor packed = at::empty({N, K / 2}, weights.options().dtype(at::kByte));
+    at::Tensor scales = at::empty({N, K / group_size}, weights.options().dtype(at::kHalf));
+    const int rc = w4a16_quantize_pack(weights.data_ptr(), (int)weights.element_size(), packed.data_ptr<uint8_t>(),
+                                       scales.data_ptr(), N, K, group_size, current_stream(weights.device()));
+    TORCH_CHECK(rc == W4A16_OK, w4a16_last_error());
+    return {packed, scales};
+}
+
 }  // namespace
 
 TORCH_LIBRARY(w4a16, m) {
     m.def("linear(Tensor activations, Tensor packed_weights, Tensor scales, int group_size) -> Tensor");
     m.def("dequantize(Tensor packed_weights, Tensor scales, int group_size) -> Tensor");
+    m.def("quantize(Tensor weights, int group_size) -> (Tensor, Tensor)");
 }
 
 TORCH_LIBRARY_IMPL(w4a16, CUDA, m) {
     m.impl("linear", &linear);
     m.impl("dequantize", &dequantize);
+    m.impl("quantize", &quantize);
 }
 
 static PyModuleDef w4a16_module = {PyModuleDef_HEAD_INIT, "_C", "W4A16 torch ops (registered on import)", -1,

@@ -80,3 +80,11 @@ def dequantize_cuda(
     """
     _require_extension()
     return torch.ops.w4a16.dequantize(packed_weights, scales, group_size)
+
+
+def quantize_cuda(weights: torch.Tensor, group_size: int = 128) -> tuple[torch.Tensor, torch.Tensor]:
+    """fp16 / fp32 weights [N, K] -> (packed uint8 [N, K / 2], fp16 scales) in
+    one pass, the bytes of ``quantize_and_pack_weights``; group_size a power of
+    two from 16 to 512, weights contiguous and 16-byte aligned."""
+    _require_extension()
+    return torch.ops.w4a16.quantize(weights, group_size)

@@ -16,6 +16,9 @@ other order or precision would produce different packed bytes.
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
+
+from nibble_amd.cuda import cuda_extension_available, quantize_cuda
 
 
 def pack_int4(quantized_weights: torch.Tensor) -> torch.Tensor:
@@ -88,6 +91,33 @@ def quantize_groupwise(
 def quantize_and_pack_weights(
     weights: torch.Tensor, group_size: int = 128
 ) -> tuple[torch.Tensor, torch.Tensor]:
-    """Quantize then pack (reference ``w4a16/quantization.py:105-113``)."""
+    """Quantize then pack (reference ``w4a16/quantization.py:105-113``).
+
+    On the GPU one kernel writes the same bytes (see ``_native``).
+    """
+    if _native(weights, group_size):
+        return quantize_cuda(weights.contiguous(), group_size)
     codes, scales = quantize_groupwise(weights, group_size)
     return pack_int4(codes), scales
+
+
+def _native(weights: torch.Tensor, group_size: int) -> bool:
+    """Whether the HIP quantizer takes these weights: a GPU matrix of the types
+    the quantizer accepts, groups of a power of two from 16 to 512 (lanes of
+    one wavefront), 16-byte aligned once contiguous. Everything else, and
+    every call that the checks of the torch ops reject, that is traced or that
+    asks for derivatives, keeps the torch ops."""
+    return (
+        type(weights) in (torch.Tensor, torch.nn.Parameter)
+        and weights.is_cuda
+        and cuda_extension_available()
+        and not torch.compiler.is_compiling()
+        and weights.dtype in (torch.float16, torch.float32)
+        and weights.ndim == 2
+        and weights.numel() > 0
+        and group_size in (16, 32, 64, 128, 256, 512)
+        and weights.shape[1] % group_size == 0
+        and not (weights.is_contiguous() and weights.data_ptr() % 16)
+        and not (weights.requires_grad and torch.is_grad_enabled())
+        and forward_ad.unpack_dual(weights).tangent is None
+    )

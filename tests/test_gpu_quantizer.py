@@ -93,3 +93,40 @@ def test_device_quantizer_wide_range_and_fp16_input(gpu):
     p, s = _device_quantize(w16, 128, gpu)
     rp, rs = oracle.quantize_and_pack(w16.astype(np.float32), 128)
     assert np.array_equal(p, rp) and np.array_equal(s.view(np.uint16), rs.view(np.uint16))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("group", [16, 32, 64, 128, 256, 512, 48, 1024])
+@pytest.mark.parametrize("n,groups", [(1, 1), (3, 5), (37, 9), (300, 7)])
+def test_device_quantizer_kernel_matches_torch_ops(gpu, dtype, group, n, groups):
+    """quantize_and_pack_weights on the device (one kernel for groups of a
+    power of two up to 512, torch ops for 48 and 1024) against the two torch
+    ops on the same tensors: last blocks that are not full, a zero group,
+    ties, infinities, NaN, and weights whose scale is subnormal or whose
+    fp16 scale overflows."""
+    from nibble_amd.quantization import pack_int4
+
+    gen = torch.Generator().manual_seed(n * 1000 + groups + group)
+    w = torch.randn((n, groups * group), generator=gen) * torch.exp(torch.rand((n, 1), generator=gen) * 12 - 8)
+    w = w.to(dtype)
+    w[0, :group] = (torch.arange(group) % 27 - 13) * 0.0625   # scale 0.8125 / 7; every half step
+    if n > 8:
+        w[1] = 0
+        w[2, 3] = float("inf")
+        w[3, 5] = float("nan")
+        w[4, :] *= torch.finfo(dtype).tiny
+        w[5, 0] = torch.finfo(dtype).max
+        w[6, :group] = (torch.arange(group) % 27 - 13) * 0.0625
+        w[6, 0] = 0.875   # scale exactly 0.125: ties
+    w = w.to(gpu)
+    print(f"[case] {dtype} {tuple(w.shape)} G={group}", flush=True)
+    for what, v in (("whole", w), ("transposed storage", w.t().contiguous().t())):
+        packed, scales = quantize_and_pack_weights(v, group)
+        codes, ref_scales = quantize_groupwise(v, group)
+        assert torch.equal(packed, pack_int4(codes)), what
+        assert torch.equal(scales.view(torch.int16), ref_scales.view(torch.int16)), what
+    if n > 8:   # rows from an odd element on: a view that is contiguous but not 16-byte aligned
+        flat = torch.cat([w.reshape(-1)[:1], w.reshape(-1)])
+        packed, scales = quantize_and_pack_weights(flat[1:].view_as(w), group)
+        ref = quantize_and_pack_weights(w, group)
+        assert torch.equal(packed, ref[0]) and torch.equal(scales.view(torch.int16), ref[1].view(torch.int16))
