@@ -80,6 +80,11 @@ int launch_gemm2(int mt, int rb, int sn, int sk, int M, const void* x, const uin
 bool gemm3_instantiated(int mt, int rb, int sn, int sk, bool paired);
 int launch_gemm3(int mt, int rb, int sn, int sk, bool paired, int M, const void* x, const uint8_t* w, const void* s,
                  void* o, int N, int K, hipStream_t stream);
+// w4a16_group.hip: group sizes 32 and 64 at M = 1..8
+bool group_fits(int64_t M, int64_t N, int64_t K, int64_t G, const void* scales);
+void group_plan(int64_t M, int64_t N, int64_t K, int* sk, int* sn, int* depth);
+int launch_group(int G, int sk, int sn, int depth, int M, const void* x, const uint8_t* w, const void* s, void* o,
+                 int N, int K, hipStream_t stream);
 }  // namespace w4a16_internal
 
 namespace {
@@ -910,10 +915,17 @@ int make_plan(const void* act, const void* packed, const void* scales, int64_t M
     const bool tuned = aligned && M <= 8;
     if (!tuned) {
         Plan p;
+        // any group size and alignment: the scalar kernel, and (max_blocks = 1)
+        // its matrix-core form for group sizes 32 and 64 at M = 1..8, on every
+        // layer that form takes (w4a16_group.hip)
         p.kernel = W4A16_KERNEL_GENERIC;
         p.rows = 4;
         p.splits = 1;
         p.unroll = 1;
+        if (aligned16(act) && aligned16(packed) && w4a16_internal::group_fits(M, N, K, G, scales)) {
+            w4a16_internal::group_plan(M, N, K, &p.splits, &p.rows, &p.unroll);
+            p.max_blocks = 1;
+        }
         *out = p;
         return W4A16_OK;
     }
@@ -1324,7 +1336,11 @@ int run_plan(const Plan& p, const void* act, const uint8_t* packed, const void* 
         case W4A16_KERNEL_GEMM32:
             return w4a16_internal::launch_gemm3(p.rows, p.max_blocks, p.unroll, p.splits, false, (int)M, x, packed, s, o,
                                                 (int)N, (int)K, st);
-        case W4A16_KERNEL_GENERIC: return launch_generic((int)M, x, packed, s, o, (int)N, (int)K, (int)G, st);
+        case W4A16_KERNEL_GENERIC:
+            if (p.max_blocks == 1 && aligned16(x) && aligned16(packed) && w4a16_internal::group_fits(M, N, K, G, s))
+                return w4a16_internal::launch_group((int)G, p.splits, p.rows, p.unroll, (int)M, x, packed, s, o, (int)N,
+                                                    (int)K, st);
+            return launch_generic((int)M, x, packed, s, o, (int)N, (int)K, (int)G, st);
         default: return fail(W4A16_ERR_CONFIG, "unknown kernel family");
     }
 }

@@ -1,0 +1,71 @@
+"""Group sizes 32 and 64 at M = 1..8 on the matrix-core form of the generic
+family (w4a16_group.hip), through the default route and every launch shape,
+against the fp32 oracle."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from _cases import assert_parity, expected, make_case
+from nibble_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _on(gpu, *tensors):
+    return [t.to(gpu) for t in tensors]
+
+
+# one run, an odd run count (a padded half pair), ragged N, rows that fill LDS (14336 at M = 8: two launches)
+@pytest.mark.parametrize("k,n", [(128, 8), (128, 5), (384, 19), (640, 250), (1024, 64), (2176, 515), (4096, 4100),
+                                 (2048, 8200), (14336, 24)])
+@pytest.mark.parametrize("group", [32, 64])
+@pytest.mark.parametrize("m", [1, 2, 4, 5, 8])
+def test_group_default_route(gpu, m, group, k, n):
+    x, p, s = make_case(m, k, n, seed=k + n + m, all_nibbles=True, group_size=group)
+    xd, pd, sd = _on(gpu, x / 8, p, s)
+    plan = _lib.plan_linear(xd.data_ptr(), pd.data_ptr(), m, n, k, group)
+    print(f"[case] M={m} K={k} N={n} G={group} {plan}", flush=True)
+    assert plan["kernel"] == "generic" and plan["max_blocks"] == 1
+    out = torch.full((m, n), float("nan"), dtype=torch.float16, device=gpu)
+    _lib.linear_f16(xd, pd, sd, out, group)
+    torch.cuda.synchronize()
+    assert_parity(out, expected(x / 8, p, s, group), f"M={m} K={k} N={n} G={group}")
+
+
+@pytest.mark.parametrize("splits,rows", [(1, 1), (1, 8), (2, 3), (4, 2), (8, 1)])
+@pytest.mark.parametrize("depth", [1, 2, 4])
+@pytest.mark.parametrize("m,group", [(1, 64), (1, 32), (3, 32), (8, 64)])
+def test_group_launch_shapes(gpu, m, group, splits, rows, depth):
+    k, n = 9 * 128, 100   # 5 run pairs, the last half padded: wavefronts with none at 8 splits
+    x, p, s = make_case(m, k, n, seed=splits + depth, group_size=group)
+    xd, pd, sd = _on(gpu, x, p, s)
+    out = torch.full((m, n), float("nan"), dtype=torch.float16, device=gpu)
+    print(f"[case] M={m} G={group} splits={splits} rows={rows} depth={depth}", flush=True)
+    _lib.linear_f16_tuned(xd, pd, sd, out, group, _lib.KERNEL_GENERIC, rows, splits, depth, 1)
+    torch.cuda.synchronize()
+    assert_parity(out, expected(x, p, s, group), f"M={m} G={group} {splits}x{rows} D={depth}")
+
+
+def test_group_scales_of_other_alignment_and_inf(gpu):
+    """Scales that are only 2-byte aligned keep the scalar kernel; a non-finite
+    scale or activation of one group reaches only its own outputs."""
+    for group in (32, 64):
+        x, p, s = make_case(2, 640, 24, seed=group, group_size=group)
+        s[3, 1] = float("inf")
+        x[1, 7] = float("inf")
+        xd, pd = _on(gpu, x, p)
+        store = torch.empty((s.numel() + 1,), dtype=torch.float16, device=gpu)
+        store[1:] = s.to(gpu).reshape(-1)
+        got = []
+        for sd in (s.to(gpu), store[1:].view_as(s)):
+            out = torch.empty((2, 24), dtype=torch.float16, device=gpu)
+            print(f"[case] G={group} scales at {sd.data_ptr() % 16}", flush=True)
+            _lib.linear_f16(xd, pd, sd, out, group)
+            torch.cuda.synchronize()
+            got.append(out.float().cpu())
+        finite = torch.isfinite(got[1])
+        assert torch.equal(finite, torch.isfinite(got[0]))
+        assert finite[0].sum() == 23 and not finite[0, 3]
+        assert torch.allclose(got[0][finite], got[1][finite], rtol=1e-3, atol=1e-3)
