@@ -448,6 +448,22 @@ __host__ __device__ constexpr int64_t gemm3_lds_bytes(int mt, int rb, int sn, in
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
+// Tile of workgroup b. Workgroups go to the 8 XCDs in turn (b % 8); each XCD
+// takes a contiguous share of the tiles, counted along the activation blocks
+// first, so the activation blocks of one weight block follow one another on
+// the same XCD and re-read those weights from its L2, and no XCD has more
+// than one tile above another: giving each XCD whole weight blocks left 66
+// tiles on some and 55 on others (M = 700, 2048 x 2 x 5632, 64 resident), a
+// second round of the whole kernel for two of them.
+__device__ __forceinline__ void xcd_tile(int b, int nblocks, int& nbk, int& mbk) {
+    const int tiles = (int)gridDim.x;
+    const int mblocks = tiles / nblocks;
+    const int x = b & 7, each = tiles >> 3, rest = tiles & 7;
+    const int t = x * each + min(x, rest) + (b >> 3);
+    nbk = t / mblocks;
+    mbk = t - nbk * mblocks;
+}
+
 template <int MT, int RB, int SN, int SK, bool PAIRED = false, int LA = 2>
 __global__ void __launch_bounds__(64 * SN * SK)
 gemm3_w4a16(const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16* __restrict__ scales,
@@ -461,11 +477,8 @@ gemm3_w4a16(const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16*
     constexpr int UPT = UNITS / T;
     constexpr int BUF = SK * 32 * MT * kGemmRow;   // halves per staging buffer
     const int b = blockIdx.x;
-    const int mblocks = (int)gridDim.x / ((nblocks + 7) & ~7);
-    const int sidx = b >> 3;
-    const int nbk = 8 * (sidx / mblocks) + (b & 7);
-    const int mbk = sidx % mblocks;
-    if (nbk >= nblocks) return;   // padding workgroup: whole workgroup, before any barrier
+    int nbk, mbk;
+    xcd_tile(b, nblocks, nbk, mbk);
 
     extern __shared__ __align__(16) uint8_t smem[];
     f16* as = reinterpret_cast<f16*>(smem);                                   // [2][SK][32 MT][kGemmRow]
@@ -476,33 +489,42 @@ gemm3_w4a16(const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16*
     const int sk = wave % SK, sn = wave / SK;
     const int G = K >> 7;
     const int R = (G + SK - 1) / SK;
-    const int RP = (R + DB - 1) / DB * DB;   // rounds run, a multiple of the ring
     const uint32_t row_bytes = (uint32_t)(K >> 1);
     const int n0 = nbk * 32 * RO * SN + sn * 32 * RO;
     const int m0 = mbk * 32 * MT;
 
-    // staging: unit u = (group gl, row, 16-byte part p) of the round
+    // staging: thread t's unit p of a round is 16 bytes (part t % 16) of row
+    // (p T mod 512 MT + t) / 16 of group p T / (512 MT): the group and the
+    // bytes it starts at are the same for the whole workgroup, so a unit's
+    // address is a scalar base that moves with the round plus an offset that
+    // does not
+    static_assert((512 * MT) % T == 0, "a unit's group does not depend on the thread");
+    constexpr int RU = 512 * MT / T;   // units per group and thread
     const uint8_t* xbase = reinterpret_cast<const uint8_t*>(x);
-    auto stage_load = [&](u32x4 (&a)[UPT], int r) {
+    uint32_t xoff[RU];
+#pragma unroll
+    for (int p = 0; p < RU; ++p)
+        xoff[p] = (uint32_t)min(m0 + ((p * T + (int)threadIdx.x) >> 4), M - 1) * (uint32_t)K * 2u +
+                  (threadIdx.x & 15u) * 16u;
+    f16* const put = as + (threadIdx.x >> 4) * kGemmRow + (threadIdx.x & 15) * 8;
+    auto stage_load = [&](u32x4 (&a)[UPT], int r, int from, int to) {
 #pragma unroll
         for (int p = 0; p < UPT; ++p) {
-            const int u = threadIdx.x + p * T;
-            const int gl = u / (32 * MT * 16), rem = u % (32 * MT * 16);
-            const int row = rem >> 4, part = rem & 15;
-            const int g = min(r * SK + gl, G - 1);
-            const uint32_t m = (uint32_t)min(m0 + row, M - 1);
-            a[p] = *reinterpret_cast<const u32x4*>(xbase + (m * (uint32_t)K + (uint32_t)g * 128u + part * 8u) * 2u);
+            if (p < from || p >= to) continue;
+            const uint8_t* base = xbase + (size_t)min(r * SK + p / RU, G - 1) * 256u;
+            a[p] = *reinterpret_cast<const u32x4*>(base + xoff[p % RU]);
         }
     };
-    auto stage_put = [&](const u32x4 (&a)[UPT], int r, int buf) {
+    // into unpack8's pair order; groups past K as zeros (v_perm selectors of the zero byte)
+    auto stage_put = [&](const u32x4 (&a)[UPT], int r, int buf, int from, int to) {
 #pragma unroll
         for (int p = 0; p < UPT; ++p) {
-            const int u = threadIdx.x + p * T;
-            const int gl = u / (32 * MT * 16), rem = u % (32 * MT * 16);
-            const int row = rem >> 4, part = rem & 15;
-            const bool live = r * SK + gl < G;
-            *reinterpret_cast<u32x4*>(as + (size_t)buf * BUF + ((size_t)gl * 32 * MT + row) * kGemmRow + part * 8) =
-                live ? a[p] : (u32x4){0u, 0u, 0u, 0u};
+            if (p < from || p >= to) continue;
+            const bool live = SK == 1 || r * SK + p / RU < G;   // SK = 1: no round holds part of one
+            const uint32_t lo = live ? 0x05040100u : 0x0C0C0C0Cu, hi = live ? 0x07060302u : 0x0C0C0C0Cu;
+            const u32x4 v = {perm(a[p].z, a[p].x, lo), perm(a[p].z, a[p].x, hi), perm(a[p].w, a[p].y, lo),
+                             perm(a[p].w, a[p].y, hi)};
+            *reinterpret_cast<u32x4*>(put + buf * BUF + (p / RU * 32 * MT + p % RU * (T / 16)) * kGemmRow) = v;
         }
     };
 
@@ -518,15 +540,21 @@ gemm3_w4a16(const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16*
         srow[t] = n * (uint32_t)G * 2u;
     }
     u32x4 wv[DB][RB][2];
-    uint32_t sv[DB][RB];
+    uint32_t sv[DB][RB], sn_[DB][RB];   // scales of this and of the next DB rounds
     auto load_w = [&](int d, int r) {
-        const uint32_t g = (uint32_t)min(r * SK + sk, G - 1);
-#pragma unroll
-        for (int t = 0; t < RB; ++t) sv[d][t] = *reinterpret_cast<const uint16_t*>(sbase + srow[t] + g * 2u);
+        const uint8_t* base = w + (size_t)min(r * SK + sk, G - 1) * 64u;
 #pragma unroll
         for (int t = 0; t < RB; ++t) {
-            wv[d][t][0] = *reinterpret_cast<const u32x4*>(w + wrow[t] + g * 64u);
-            wv[d][t][1] = *reinterpret_cast<const u32x4*>(w + wrow[t] + g * 64u + 16u);
+            wv[d][t][0] = *reinterpret_cast<const u32x4*>(base + wrow[t]);
+            wv[d][t][1] = *reinterpret_cast<const u32x4*>(base + wrow[t] + 16);
+        }
+    };
+    auto load_s = [&](uint32_t (&to)[DB][RB], int r) {
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+            const uint8_t* base = sbase + 2 * (size_t)min((r + d) * SK + sk, G - 1);
+#pragma unroll
+            for (int t = 0; t < RB; ++t) to[d][t] = *reinterpret_cast<const uint16_t*>(base + srow[t]);
         }
     };
 
@@ -538,79 +566,121 @@ gemm3_w4a16(const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16*
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[t][r][e] = 0.0f;
 
-    const f16x2 mul = {(f16)1.0f, (f16)0.0625f};
-    const f16x2 off = {(f16)-1032.0f, (f16)-72.0f};
-    auto compute = [&](int d, int buf) {
-        const f16* ab = as + (size_t)buf * BUF + (size_t)sk * 32 * MT * kGemmRow;
-        // A fragments one step ahead: step st + 1's LDS reads are in flight
-        // while step st decodes and runs its MFMAs
-        u32x4 afn[MT];
+    // A fragments of step st of a staged round, and the round's decoded weights
+    auto read_a = [&](u32x4 (&af)[MT], int buf, int st) {
+        const f16* ab = as + (size_t)buf * BUF + (size_t)sk * 32 * MT * kGemmRow + 64 * h + 8 * st;
 #pragma unroll
-        for (int t = 0; t < MT; ++t) afn[t] = *reinterpret_cast<const u32x4*>(ab + (32 * t + c) * kGemmRow + 64 * h);
+        for (int t = 0; t < MT; ++t) af[t] = *reinterpret_cast<const u32x4*>(ab + (32 * t + c) * kGemmRow);
+    };
+    auto decode = [&](f16x8 (&bt)[RB], int d, int st) {
 #pragma unroll
-        for (int st = 0; st < 8; ++st) {
-            u32x4 af[MT];
-#pragma unroll
-            for (int t = 0; t < MT; ++t) af[t] = afn[t];
-            if (st < 7) {
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-                    afn[t] = *reinterpret_cast<const u32x4*>(ab + (32 * t + c) * kGemmRow + 64 * h + 8 * (st + 1));
-            }
-#pragma unroll
-            for (int r = 0; r < RB; ++r) {
-                const f16 sc = __builtin_bit_cast(f16, (uint16_t)sv[d][r]);
-                const f16x2 sc2 = {sc, sc};
-                const uint32_t word = wv[d][r][st >> 2][st & 3];
-                f16x2 pr[4];
-#pragma unroll
-                for (int by = 0; by < 4; ++by) {
-                    const uint32_t sel = (0x0Cu << 24) | ((uint32_t)by << 16) | (0x0Cu << 8) | (uint32_t)by;
-                    const uint32_t v = __builtin_amdgcn_bitop3_b32(perm(word, word, sel), 0x00F0000Fu, 0x64806408u,
-                                                                   0x6A);
-                    pr[by] = __builtin_elementwise_fma(as_f16x2(v), mul, off) * sc2;
-                }
-                const f16x8 bt = __builtin_bit_cast(
-                    f16x8, (u32x4){as_u32(pr[0]), as_u32(pr[1]), as_u32(pr[2]), as_u32(pr[3])});
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-                    acc[t][r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, af[t]), bt,
-                                                                       acc[t][r], 0, 0, 0);
-            }
+        for (int r = 0; r < RB; ++r) {
+            const f16 sc = __builtin_bit_cast(f16, (uint16_t)sv[d][r]);
+            const f16x2 sc2 = {sc, sc};
+            const Codes8 cw = unpack8(wv[d][r][st >> 2][st & 3]);
+            bt[r] = __builtin_bit_cast(f16x8, (u32x4){as_u32(cw.p[0] * sc2), as_u32(cw.p[1] * sc2),
+                                                      as_u32(cw.p[2] * sc2), as_u32(cw.p[3] * sc2)});
         }
     };
 
-    // prologue: round 0 staged, round 1 requested, the ring's first DB rounds
-    // of weights requested. Staging runs two rounds ahead: round r's loop
-    // requests round r + 2 into the register set round r came from and puts
-    // round r + 1 (requested a round earlier) into LDS, so a staging load has
-    // two rounds of MFMAs to arrive.
-    // (LA = 1: round r requests round r + 1 and puts it after its MFMAs, for
-    // shapes whose registers only hold one staging set.)
+    // Software pipeline. A step's MFMAs run on fragments read and weights
+    // decoded during the step before it, so that the VALU work and the LDS
+    // reads issue in the shadow of the matrix instructions (32 cycles each).
+    // The next round is put into the other LDS buffer during steps 1..5; the
+    // round's only barrier stands before its last step, which then reads the
+    // next round's first fragments: by then every wavefront holds its last
+    // fragments of this round in registers. A unit's registers are reloaded
+    // right after their put, LA rounds ahead of the next one. Weights are
+    // requested for two rounds at a time (both 64-byte halves of a cache line)
+    // and scales for DB rounds, so that a line that several rounds use comes
+    // from the L2 once.
     static_assert(LA == 1 || LA == 2, "staging runs one or two rounds ahead");
+    static_assert(DB == 4, "the staging register sets and weight pairs alternate within the ring");
     u32x4 a[LA][UPT];
-    stage_load(a[0], 0);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int d = 0; d < DB; ++d) load_w(d, d);
-    if constexpr (LA == 2) stage_load(a[LA - 1], 1);
-    __builtin_amdgcn_sched_barrier(0);
-    stage_put(a[0], 0, 0);
-    __syncthreads();
-    static_assert(DB % 2 == 0, "the staging register sets alternate within the weight ring");
-    for (int r0 = 0; r0 < RP; r0 += DB) {
-#pragma unroll
-        for (int d = 0; d < DB; ++d) {
-            const int r = r0 + d;
-            // past the last round: clamped, staged as zeros, never read
-            if constexpr (LA == 2) stage_load(a[d & 1], r + 2);
-            else stage_load(a[0], r + 1);
-            compute(d, r & 1);
-            load_w(d, r + DB);
-            stage_put(a[LA == 2 ? (d + 1) & 1 : 0], r + 1, (r + 1) & 1);
-            __syncthreads();
-        }
+    {
+        // rounds 0 .. LA of the activations and the weight ring in one go: one memory latency, not one per round
+        u32x4 first[UPT];
+        stage_load(first, 0, 0, UPT);
+        __builtin_amdgcn_sched_barrier(0);
+        load_s(sv, 0);
+        load_w(0, 0);
+        load_w(1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        stage_load(a[LA == 2 ? 1 : 0], 1, 0, UPT);
+        if constexpr (LA == 2) stage_load(a[0], 2, 0, UPT);
+        load_w(2, 2);
+        load_w(3, 3);
+        __builtin_amdgcn_sched_barrier(0);
+        stage_put(first, 0, 0, 0, UPT);
     }
+    __syncthreads();
+    u32x4 af[MT];
+    f16x8 bt[RB];
+    read_a(af, 0, 0);
+    decode(bt, 0, 0);
+    constexpr int NM = MT * RB;              // MFMAs per step
+    constexpr int PUTS = (UPT + 4) / 5;      // units put per step, steps 1..5
+    // round r = r0 + d on ring slot d; refill: request the rounds ahead (the last rounds of a row need none)
+    auto round = [&](int d, int r, bool refill) __attribute__((always_inline)) {
+        const int buf = d & 1;
+        if (refill && d == 0) load_s(sn_, r + DB);
+#pragma unroll
+        for (int st = 0; st < 8; ++st) {
+            u32x4 an[MT];
+            f16x8 bn[RB];
+            if (st < 7) {
+                read_a(an, buf, st + 1);
+                decode(bn, d, st + 1);
+            } else {
+                __syncthreads();
+                read_a(an, buf ^ 1, 0);
+                if (d == DB - 1) {
+#pragma unroll
+                    for (int e = 0; e < DB; ++e)
+#pragma unroll
+                        for (int t = 0; t < RB; ++t) sv[e][t] = sn_[e][t];
+                }
+                decode(bn, (d + 1) % DB, 0);
+                if (refill && (d & 1)) {
+                    load_w(d - 1, r - 1 + DB);
+                    load_w(d, r + DB);
+                }
+            }
+            if (st >= 1 && st <= 5) {
+                u32x4(&set)[UPT] = a[LA == 2 ? (d + 1) & 1 : 0];
+                stage_put(set, r + 1, buf ^ 1, (st - 1) * PUTS, st * PUTS);
+                if (refill || LA == 1) stage_load(set, r + 1 + LA, (st - 1) * PUTS, st * PUTS);
+            }
+#pragma unroll
+            for (int rr = 0; rr < RB; ++rr)
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    acc[t][rr] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, af[t]), bt[rr],
+                                                                        acc[t][rr], 0, 0, 0);
+            // one LDS read and an even share of the decode after each MFMA
+#pragma unroll
+            for (int i = 0; i < NM; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                           // MFMA
+                if (i < MT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);               // LDS read
+                __builtin_amdgcn_sched_group_barrier(0x002, (14 * RB + NM - 1) / NM, 0);     // VALU
+            }
+#pragma unroll
+            for (int t = 0; t < MT; ++t) af[t] = an[t];
+#pragma unroll
+            for (int rr = 0; rr < RB; ++rr) bt[rr] = bn[rr];
+        }
+    };
+    int r0 = 0;
+    for (; r0 + DB <= R; r0 += DB) {   // no branch around a load: joins would make the compiler wait for all of them
+        round(0, r0, true);
+        round(1, r0 + 1, true);
+        round(2, r0 + 2, true);
+        round(3, r0 + 3, true);
+    }
+    if (r0 < R) round(0, r0, false);
+    if (r0 + 1 < R) round(1, r0 + 1, false);
+    if (r0 + 2 < R) round(2, r0 + 2, false);
+    __syncthreads();   // the staging buffers become the reduction's
 
     // SK partial tiles: wavefronts sk > 0 write, sk = 0 sums in order
     if (SK > 1) {

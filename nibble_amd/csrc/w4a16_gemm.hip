@@ -275,7 +275,7 @@ int launch_gemm3(int mt, int rb, int sn, int sk, bool paired, int M, const void*
     const int cols = (paired ? 16 : 32) * rb * sn;   // output columns per workgroup
     const int nblocks = (N + cols - 1) / cols;
     const int mblocks = (M + 32 * mt - 1) / (32 * mt);
-    const int64_t grid = (int64_t)((nblocks + 7) & ~7) * mblocks;
+    const int64_t grid = (int64_t)nblocks * mblocks;
     if (grid > INT32_MAX) return fail(W4A16_ERR_TOO_LARGE, "32x32 GEMM kernel: too many workgroups");
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * sn * sk), (size_t)lds, stream,
                        static_cast<const w4a16::f16*>(x), w, static_cast<const w4a16::f16*>(s),
