@@ -100,7 +100,8 @@ int64_t w4a16_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t gr
  * M = 3..8 layers of K = 28672 (N = 4096..8192) and M = 5..8 layers of
  * K = 8192 with N >= 16384 the paired ring kernel over K slices; the fp32
  * partial sums are added in slice
- * order by a second launch. workspace == NULL routes exactly as w4a16_linear_f16;
+ * order by a second launch; M > 16 takes the GEMM shape of the least estimated
+ * time (no workspace bytes used). workspace == NULL routes exactly as w4a16_linear_f16;
  * a smaller non-NULL workspace is W4A16_ERR_CONFIG. The torch op
  * w4a16::linear (reference csrc/int4_linear.cpp:16-28) calls this entry
  * point with a workspace from the caching allocator.

@@ -544,6 +544,62 @@ bool plan_gemm32_silu(int64_t M, int64_t inter, int64_t K, Plan* out) {
     return false;
 }
 
+// Prompt rows where the caller leaves the route to the library
+// (w4a16_linear_ws_f16 with a workspace pointer, the torch op, the fused
+// prefill launches): the GEMM shape with the least estimated time. A launch
+// of t tiles on 256 CUs takes about (us at K / 1024 = k) a k + b for up to 256
+// tiles; past that a further round, of which a shape that fits twice on a CU
+// hides the part of `hide` that its last round leaves empty. a, b and hide
+// from a sweep of every shape over M 24..1024 on eight layers (graph timing,
+// rotated weights), which this picks the fastest of, or one within 6%, in all
+// of 64 cases. Where the fixed thresholds above lose: M = 384, 14336 x
+// 4096 77 against 135 us; M = 200 56 against 70; M = 384, 5632 x 2048 23.4
+// against 31.5; M = 700, 2048 x 5632 26 against 35; M = 700, 4096 x 14336 110
+// against 126.
+struct GemmCost {
+    int mt, rb, sn, sk;
+    double a, b, hide;
+};
+
+double gemm_cost(const GemmCost& c, int tile, int64_t M, int64_t N, int64_t K) {
+    const int64_t rows = (int64_t)tile * c.mt, cols = (int64_t)tile * c.rb * c.sn;
+    const int64_t tiles = ((N + cols - 1) / cols) * ((M + rows - 1) / rows);
+    const double rounds = (double)((tiles + 255) / 256), last = (double)((tiles - 1) % 256 + 1) / 256.0;
+    return (rounds - (rounds > 1 ? c.hide * (1.0 - last) : 0.0)) * (c.a * (double)K / 1024.0 + c.b);
+}
+
+bool plan_prompt(int64_t M, int64_t N, int64_t K, Plan* p) {
+    static const GemmCost k32[] = {{4, 2, 4, 1, 14.5, 3.0, 0.0}, {4, 1, 4, 1, 9.3, 1.5, 0.35}, {2, 2, 4, 1, 10.3, 3.5, 0.35},
+                                   {2, 1, 4, 2, 5.4, 4.0, 0.35}, {2, 1, 2, 4, 3.45, 6.2, 0.0}, {2, 1, 1, 4, 2.6, 5.5, 0.0}};
+    static const GemmCost k16[] = {{1, 1, 1, 4, 1.1, 2.7, 0.35}, {1, 2, 1, 4, 1.7, 2.6, 0.35}, {1, 4, 1, 4, 2.8, 2.7, 0.35},
+                                   {2, 1, 1, 4, 2.0, 2.5, 0.35}, {2, 2, 1, 4, 2.75, 2.3, 0.35}, {2, 4, 1, 4, 3.55, 3.4, 0.35},
+                                   {4, 4, 1, 4, 4.6, 6.0, 0.35}};
+    if (M <= 16 || K < 1024) return false;   // below the sweep: the thresholds above
+    double best = 1e30;
+    for (const auto& c : k16) {
+        const double t = gemm_cost(c, 16, M, N, K);
+        if (16 * (c.mt - 1) >= M || t >= best || !w4a16_internal::gemm_instantiated(c.mt, c.rb, c.sk)) continue;
+        best = t;
+        *p = Plan();
+        p->kernel = W4A16_KERNEL_GEMM;
+        p->rows = c.mt;
+        p->max_blocks = c.rb;
+        p->splits = c.sk;
+    }
+    for (const auto& c : k32) {
+        const double t = gemm_cost(c, 32, M, N, K);
+        if (t >= best || !w4a16_internal::gemm3_instantiated(c.mt, c.rb, c.sn, c.sk, false)) continue;
+        best = t;
+        *p = Plan();
+        p->kernel = W4A16_KERNEL_GEMM32;
+        p->rows = c.mt;
+        p->max_blocks = c.rb;
+        p->unroll = c.sn;
+        p->splits = c.sk;
+    }
+    return true;
+}
+
 // Largest M the dispatcher sends to the GEMM kernel.
 constexpr int64_t kGemmMaxM = 1 << 20;
 
@@ -909,6 +965,7 @@ int make_plan(const void* act, const void* packed, const void* scales, int64_t M
     // weights its staged 32x32 form, and the staged 16x16 form on longer rows
     // of wide layers from M = 128
     if (aligned && M > 8 && gemm_fits(M, N, K)) {
+        if (workspace && plan_prompt(M, N, K, out)) return W4A16_OK;
         if (!plan_gemm32(M, N, K, out)) *out = gemm_lds_route(M, N, K) ? plan_gemm_lds(M, N, K) : plan_gemm(M, N, K);
         return W4A16_OK;
     }

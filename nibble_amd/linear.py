@@ -44,6 +44,12 @@ FUSED_MAX_ROWS = 8
 # 131 us, 2048 x 11264 75 against 69) and on most layers at M = 2048, so
 # longer prompts keep it.
 NATIVE_GEMM_MAX_ROWS = 512
+# Layers of at most this many weights keep the W4A16 GEMM up to twice those
+# rows: 2048 x 5632 at M = 600 22.9 against 35.6 us, 5632 x 2048 at M = 1024
+# 35.4 against 46.9, 2048 x 11264 at M = 1024 61.0 against 69.4; larger layers
+# lose some (4096 x 14336 at M = 600 104.8 against 96.8, 4096 x 6144 at M = 768
+# 63.2 against 60.9).
+NATIVE_GEMM_SMALL_LAYER = 24_000_000
 
 
 class QuantizedLinear(torch.nn.Module):
@@ -130,6 +136,12 @@ class QuantizedLinear(torch.nn.Module):
             f"group_size={self.group_size}, bias={self.bias is not None}, fused={self.fused}"
         )
 
+    def _native_rows(self) -> int:
+        """Most prompt rows that take the W4A16 GEMM: ``native_max_rows``, twice
+        its default on small layers (a value set by the caller stands as it is)."""
+        small = self.in_features * self.out_features <= NATIVE_GEMM_SMALL_LAYER
+        return self.native_max_rows * (2 if small and self.native_max_rows == NATIVE_GEMM_MAX_ROWS else 1)
+
     def _dequant_linear(self, activations: torch.Tensor) -> torch.Tensor:
         """fp16 weight matrix from the packed codes, then a dense GEMM."""
         if self.packed_weights.is_cuda:
@@ -161,7 +173,7 @@ class QuantizedLinear(torch.nn.Module):
                 raise ValueError("scales must be contiguous")
             if self.fused and rows <= FUSED_MAX_ROWS:
                 out = linear_cuda(flat, self.packed_weights, self.scales, self.group_size)
-            elif self.fused and self.group_size == 128 and rows <= self.native_max_rows:
+            elif self.fused and self.group_size == 128 and rows <= self._native_rows():
                 out = linear_cuda(flat, self.packed_weights, self.scales, self.group_size)
             elif self.group_size % 32 == 0:
                 out = self._dequant_linear(flat)
