@@ -35,25 +35,32 @@ namespace w4a16 {
 //      uses its own copy of slot p (never the cache line another workgroup
 //      is writing);
 //   2. slots 0..p in chunks of 64, wavefront w taking chunks w, w + WA, ...:
-//      lane t holds slot c0 + t's key row (8 16-byte loads, requested before
-//      any is used) and its score q.k / 8 in fp32; the chunk's value rows go
-//      to the wavefront's LDS tile (coalesced 16-byte loads, rows past p
-//      zeroed); an online softmax (running max, rescaled sum and output; DPP
-//      reductions) folds the chunk in, and lane d accumulates
-//      sum_t prob_t v_t[d]. The next chunk's rows are requested before the
-//      current chunk's reductions;
-//   3. the WA partial states (max m_w, sum l_w, output o_w) combine as
-//      out[d] = sum_w o_w[d] e^(m_w - M) / sum_w l_w e^(m_w - M), rounded to
-//      fp16 (a wavefront with no chunk has l_w = 0 and drops out).
+//      lanes 8 r .. 8 r + 7 hold rows r, r + 8, .. of the chunk, 8 elements a
+//      lane, so every load instruction of keys and values reads 8 whole rows
+//      (1 KiB); a row's score q.k / 8 is four v_dot2 a lane and a sum over its
+//      8 lanes (DPP), in fp32; an online softmax (running max, rescaled sum
+//      and output; DPP reductions) folds the chunk in, each lane keeping its
+//      8 elements of the output over its rows. The next chunk's rows are
+//      requested as soon as the current chunk's are used;
+//   3. the rows of a wavefront, then the WA partial states (max m_w, sum l_w,
+//      output o_w) combine through LDS as out[d] = sum_w o_w[d] e^(m_w - M) /
+//      sum_w l_w e^(m_w - M), rounded to fp16 (a wavefront with no chunk has
+//      l_w = 0 and drops out).
 // Slots past p get weight exactly 0. A position outside [0, S) writes NaN
 // to the head's output and touches no cache slot. Every load that does not
 // depend on the position (cache rows of each wavefront's first chunk, q, k,
 // v) is requested before the position arrives.
 // ---------------------------------------------------------------------------
 // SPLIT: workgroup (hq, s) of gridDim.y attends a share of the slots 0 .. p
-// (64-slot aligned, the shares in slot order) and writes its unnormalised
-// state to partial[hq][s] = {max, sum, acc[64]} for decode_attention_merge;
-// only share 0 appends the new k / v rows.
+// (chunks s, s + gridDim.y, ..: which ones does not depend on the position,
+// so the first of each wavefront is requested before it arrives) and writes
+// its unnormalised state to partial[hq][s] = {max, sum, acc[64]} for
+// decode_attention_merge; only share 0 appends the new k / v rows.
+// Bound: a chain of latencies (launch, position, first rows, merge launch),
+// not bytes. Graph timing, 32 / 4 heads, against keys read a row per lane and
+// values through LDS: one workgroup per head 5.7 against 7.5 us at position
+// 500 of 512 slots, 9.2 against 13.6 at 1500 of 2048; split in 8 with the
+// merge 8.2 against 8.9 at 1500, 6.9 against 8.0 at 256.
 template <int WA, bool SPLIT>
 __global__ void __launch_bounds__(64 * WA)
 decode_attention(const f16* __restrict__ qkv, f16* __restrict__ k_cache, f16* __restrict__ v_cache,
@@ -62,11 +69,10 @@ decode_attention(const f16* __restrict__ qkv, f16* __restrict__ k_cache, f16* __
                  float* __restrict__ partial) {
     static_assert(!SPLIT || WA > 1, "the split form merges its wavefronts through LDS");
     constexpr int D = 64;
-    __shared__ __align__(16) float qs_all[WA][D];
+    __shared__ __align__(16) f16 qnew_all[WA][D];
     __shared__ __align__(16) f16 knew_all[WA][D];
     __shared__ __align__(16) f16 vnew_all[WA][D];
-    __shared__ __align__(16) float probs[WA][64];
-    __shared__ __align__(16) f16 vt[WA][64 * D];
+    __shared__ __align__(16) float racc[WA][8][D];   // a wavefront's outputs by row of 8 lanes
     __shared__ float wmax[WA], wsum[WA];
     __shared__ float wacc[WA][D];
 
@@ -80,32 +86,20 @@ decode_attention(const f16* __restrict__ qkv, f16* __restrict__ k_cache, f16* __
     const f16* kc = k_cache + (size_t)hk * S * D;
     const f16* vc = v_cache + (size_t)hk * S * D;
 
-    auto load_k = [&](u32x4 (&kr)[8], int c0) {
-        const u32x4* row = reinterpret_cast<const u32x4*>(kc + (size_t)min(c0 + lane, S - 1) * D);
+    const int row0 = lane >> 3, col = lane & 7;   // rows row0 + 8 i of a chunk, elements 8 col .. + 7
+    auto load_rows = [&](u32x4 (&r)[8], const f16* cache, int c0) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) kr[e] = row[e];
-    };
-    auto load_v = [&](u32x4 (&vr)[8], int c0) {
-        // lane l: rows c0 + l/8 + 8 i, 16-byte column block l % 8
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int t = min(c0 + (lane >> 3) + 8 * i, S - 1);
-            vr[i] = reinterpret_cast<const u32x4*>(vc + (size_t)t * D)[lane & 7];
-        }
+        for (int i = 0; i < 8; ++i)
+            r[i] = reinterpret_cast<const u32x4*>(cache + (size_t)min(c0 + row0 + 8 * i, S - 1) * D)[col];
     };
     u32x4 kr[8], vr[8];
-    int c0 = 64 * wave;
-    int end = 0;   // slots c0 .. end - 1 (set below for the unsplit form)
-    if constexpr (SPLIT) {
-        const int pe = (p64 >= 0 && p64 < S) ? (int)p64 : 0;
-        // at least 3 chunks per share: shorter contexts use fewer shares
-        const int per = max(((pe + (int)gridDim.y) / (int)gridDim.y + 63) & ~63, 192);
-        const int lo = min((int)blockIdx.y * per, pe + 1);
-        c0 += lo;
-        end = min(lo + per, pe + 1);
+    const int step = SPLIT ? 64 * WA * (int)gridDim.y : 64 * WA;
+    int c0 = SPLIT ? 64 * (wave * (int)gridDim.y + (int)blockIdx.y) : 64 * wave;
+    // the split form's first wavefront only: the others' chunks may lie past the position
+    if (!SPLIT || wave == 0) {
+        load_rows(kr, kc, c0);
+        load_rows(vr, vc, c0);
     }
-    load_k(kr, c0);
-    load_v(vr, c0);
     const f16* q = qkv + (size_t)hq * D;
     const f16* k = qkv + (size_t)num_heads * D + (size_t)hk * D;
     const f16* v = qkv + (size_t)(num_heads + num_kv) * D + (size_t)hk * D;
@@ -115,6 +109,10 @@ decode_attention(const f16* __restrict__ qkv, f16* __restrict__ k_cache, f16* __
 
     const bool valid = p64 >= 0 && p64 < S;
     const int p = valid ? (int)p64 : 0;
+    if (SPLIT && wave > 0 && c0 <= p) {
+        load_rows(kr, kc, c0);
+        load_rows(vr, vc, c0);
+    }
     const float c = cos_table[(size_t)p * (D / 2) + (lane & 31)];
     const float s = sin_table[(size_t)p * (D / 2) + (lane & 31)];
     const float qa = (float)qa16, qb = (float)qb16, ka = (float)ka16, kb = (float)kb16;
@@ -122,10 +120,10 @@ decode_attention(const f16* __restrict__ qkv, f16* __restrict__ k_cache, f16* __
     const float kro = lane < 32 ? ka * c - kb * s : ka * c + kb * s;
     const f16 q16 = (f16)qr, k16 = (f16)kro;
     // every wavefront keeps its own copy (no branch the loads above could sink into)
-    float* qs = qs_all[wave];
+    f16* qnew = qnew_all[wave];
     f16* knew = knew_all[wave];
     f16* vnew = vnew_all[wave];
-    qs[lane] = (float)q16;
+    qnew[lane] = q16;
     knew[lane] = k16;
     vnew[lane] = v16;
     if (valid && wave == 0 && hq % group == 0 && (!SPLIT || blockIdx.y == 0)) {
@@ -137,66 +135,67 @@ decode_attention(const f16* __restrict__ qkv, f16* __restrict__ k_cache, f16* __
         if (!SPLIT && wave == 0) out[(size_t)hq * D + lane] = (f16)__builtin_nanf("");
         return;
     }
-    if constexpr (!SPLIT) end = p + 1;
+    const int end = p + 1;
+    const u32x4 qv = reinterpret_cast<const u32x4*>(qnew)[col];
 
-    float run_max = -__builtin_inff(), run_sum = 0.0f, acc = 0.0f;
-    f16* my_vt = vt[wave];
-    float* my_probs = probs[wave];
-    for (; c0 < end; c0 += 64 * WA) {
-        const int t = c0 + lane;
-        float dot = 0.0f;
-        if (t == p) {
+    float run_max = -__builtin_inff(), run_sum = 0.0f;
+    float o[8];
 #pragma unroll
-            for (int e = 0; e < D; ++e) dot = __builtin_fmaf(qs[e], (float)knew[e], dot);
-        } else {
+    for (int e = 0; e < 8; ++e) o[e] = 0.0f;
+    for (; c0 < end; c0 += step) {
+        if (c0 + 64 >= end) {   // the chunk of slot p, and of rows past it: nothing read from those is used
+            const u32x4 kn = reinterpret_cast<const u32x4*>(knew)[col], vn = reinterpret_cast<const u32x4*>(vnew)[col];
+            const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-#pragma unroll
-                for (int w2 = 0; w2 < 4; ++w2) {
-                    const f16x2 h = as_f16x2(kr[e][w2]);
-                    dot = __builtin_fmaf(qs[e * 8 + 2 * w2], (float)h.x, dot);
-                    dot = __builtin_fmaf(qs[e * 8 + 2 * w2 + 1], (float)h.y, dot);
-                }
+            for (int i = 0; i < 8; ++i) {
+                const int slot = c0 + row0 + 8 * i;
+                kr[i] = slot == p ? kn : kr[i];
+                vr[i] = slot == p ? vn : slot > p ? zero : vr[i];
             }
         }
-        const float score = t < end ? dot * 0.125f : -__builtin_inff();
-        // value rows of the chunk to LDS: rows past p zeroed, slot p from vnew
+        float sc[8], cmax = -__builtin_inff();
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const int row = (lane >> 3) + 8 * i;
-            const int slot = c0 + row;
-            u32x4 val = vr[i];
-            if (slot == p) val = reinterpret_cast<const u32x4*>(vnew)[lane & 7];
-            if (slot >= end) val = (u32x4){0u, 0u, 0u, 0u};
-            reinterpret_cast<u32x4*>(my_vt + row * D)[lane & 7] = val;
-        }
-        // next chunk's rows requested before this chunk's reductions
-        const int next = c0 + 64 * WA;
-        if (next < end) {
-            load_k(kr, next);
-            load_v(vr, next);
-        }
-        const float cmax = wave_max(score);
-        const float new_max = fmaxf(run_max, cmax);
-        const float pr = t < end ? expf(score - new_max) : 0.0f;
-        const float psum = wave_sum(pr);
-        const float rescale = expf(run_max - new_max);   // 0 on the first chunk
-        my_probs[lane] = pr;
-        wave_lds_sync();
-        float part = 0.0f;
+            float dot = 0.0f;
 #pragma unroll
-        for (int r4 = 0; r4 < 16; ++r4) {
-            const f32x4 pp = reinterpret_cast<const f32x4*>(my_probs)[r4];
-            part = __builtin_fmaf(pp.x, (float)my_vt[(4 * r4 + 0) * D + lane], part);
-            part = __builtin_fmaf(pp.y, (float)my_vt[(4 * r4 + 1) * D + lane], part);
-            part = __builtin_fmaf(pp.z, (float)my_vt[(4 * r4 + 2) * D + lane], part);
-            part = __builtin_fmaf(pp.w, (float)my_vt[(4 * r4 + 3) * D + lane], part);
+            for (int w2 = 0; w2 < 4; ++w2)
+                dot = __builtin_amdgcn_fdot2(as_f16x2(kr[i][w2]), as_f16x2(qv[w2]), dot, false);
+            dot += dpp<0xB1>(dot);    // quad_perm [1,0,3,2]
+            dot += dpp<0x4E>(dot);    // quad_perm [2,3,0,1]
+            dot += dpp<0x141>(dot);   // row_half_mirror: the row's 8 lanes
+            sc[i] = c0 + row0 + 8 * i < end ? dot * 0.125f : -__builtin_inff();
+            cmax = fmaxf(cmax, sc[i]);
         }
-        wave_lds_sync();
-        acc = acc * rescale + part;
-        run_sum = run_sum * rescale + psum;
+        const int next = c0 + step;
+        if (next < end) load_rows(kr, kc, next);
+        cmax = wave_max(cmax);
+        const float new_max = fmaxf(run_max, cmax);
+        const float rescale = expf(run_max - new_max);   // 0 on the first chunk
+        float psum = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] *= rescale;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float pr = c0 + row0 + 8 * i < end ? expf(sc[i] - new_max) : 0.0f;
+            psum += pr;
+#pragma unroll
+            for (int w2 = 0; w2 < 4; ++w2) {
+                const f16x2 h = as_f16x2(vr[i][w2]);
+                o[2 * w2] = __builtin_fmaf(pr, (float)h.x, o[2 * w2]);
+                o[2 * w2 + 1] = __builtin_fmaf(pr, (float)h.y, o[2 * w2 + 1]);
+            }
+        }
+        if (next < end) load_rows(vr, vc, next);
+        run_sum = run_sum * rescale + 0.125f * wave_sum(psum);   // 8 lanes hold each row
         run_max = new_max;
     }
+    // the rows of this wavefront
+    reinterpret_cast<f32x4*>(racc[wave][row0])[2 * col] = (f32x4){o[0], o[1], o[2], o[3]};
+    reinterpret_cast<f32x4*>(racc[wave][row0])[2 * col + 1] = (f32x4){o[4], o[5], o[6], o[7]};
+    wave_lds_sync();
+    float acc = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) acc += racc[wave][r][lane];
     if constexpr (WA == 1) {
         out[(size_t)hq * D + lane] = (f16)(acc / run_sum);
         return;
@@ -1587,6 +1586,8 @@ int launch_attention_o(const void* qkv, void* k_cache, void* v_cache, const floa
 
 }  // namespace
 
+constexpr int64_t kSplitMinSlots = 1024;   // caches of at most this many slots are not split
+
 extern "C" {
 
 int w4a16_decode_attention_f16(const void* qkv, void* k_cache, void* v_cache, const float* cos_table,
@@ -1635,6 +1636,13 @@ int w4a16_decode_attention_split_f16(const void* qkv, void* k_cache, void* v_cac
         !aligned(workspace, 4))
         return fail(W4A16_ERR_ALIGNMENT,
                     "split attention: caches 16-byte aligned, fp16 buffers 2-byte, workspace 4-byte aligned");
+    // caches of up to 1024 slots: one workgroup per head is faster than two
+    // launches at every position (32 / 4 heads, us: position 500 5.6 against
+    // 7.7, 1000 7.5 against 7.7); on longer ones it loses from about position
+    // 1400 on (2048 slots, position 2047: 11.1 against 9.0)
+    if (max_seq_len <= kSplitMinSlots)
+        return w4a16_decode_attention_f16(qkv, k_cache, v_cache, cos_table, sin_table, position, output, num_heads,
+                                          num_kv_heads, head_dim, max_seq_len, stream);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const auto skern = w4a16::decode_attention<4, true>;
     hipLaunchKernelGGL(skern, dim3((unsigned)num_heads, (unsigned)splits), dim3(256), 0,

@@ -206,6 +206,29 @@ def test_decode_attention_split(gpu, heads, kv, pos, splits):
     assert torch.allclose(kg[:, pos].float(), k_new.float(), rtol=2 ** -10, atol=2 ** -14)
 
 
+@pytest.mark.parametrize("heads,kv", [(32, 4), (4, 2)])
+@pytest.mark.parametrize("pos,S", [(1023, 1024), (0, 1025), (63, 1100), (64, 1100), (1024, 1025)])
+@pytest.mark.parametrize("splits", [1, 3, 8, 64])
+def test_decode_attention_split_long_caches(gpu, heads, kv, pos, S, splits):
+    """Caches around 1024 slots, the most that keep one workgroup per head, and
+    past it, where the split form runs its two launches: positions at the edges
+    of a 64-slot chunk and of the cache, more shares than chunks, one share
+    with several chunks a wavefront."""
+    qkv, k_cache, v_cache, cos, sin, ref, k_new, v_new = _decode_case(heads, kv, pos, S, pos + heads + splits)
+    kd, vd = k_cache.to(gpu), v_cache.to(gpu)
+    out = torch.empty((heads * 64,), dtype=torch.float16, device=gpu)
+    ws = torch.full((heads * splits * 66,), float("nan"), dtype=torch.float32, device=gpu)
+    position = torch.tensor([pos], dtype=torch.int64, device=gpu)
+    print(f"[case] split attention heads={heads} kv={kv} pos={pos} S={S} splits={splits}", flush=True)
+    _lib.decode_attention_split_f16(qkv.to(gpu), kd, vd, cos.to(gpu), sin.to(gpu), position, out, heads, kv,
+                                    splits, ws)
+    torch.cuda.synchronize()
+    err = (out.double().cpu() - ref).abs()
+    assert torch.all(err <= 2e-3 + 1e-2 * ref.abs()), float(err.max())   # the bound of the test above
+    assert torch.equal(vd[:, pos].cpu(), v_new)
+    assert torch.allclose(kd[:, pos].cpu().float(), k_new.float(), rtol=2 ** -10, atol=2 ** -14)
+
+
 def test_decode_attention_split_out_of_range_and_rejects(gpu):
     S, heads, kv = 256, 8, 2
     qkv = torch.randn(((heads + 2 * kv) * 64,)).to(torch.float16).to(gpu)
