@@ -600,6 +600,12 @@ bool plan_prompt(int64_t M, int64_t N, int64_t K, Plan* p) {
     return true;
 }
 
+// Outputs of w4a16_dequantize_f16 past this many bytes (the Infinity Cache,
+// 256 MB) go out with non-temporal stores; a smaller one is mostly read next,
+// by the caller's GEMM (14336 x 4096, then 2048 rows: 213 us with plain
+// stores, 227 with non-temporal ones).
+constexpr int64_t kDequantStreamBytes = 256 << 20;
+
 // Largest M the dispatcher sends to the GEMM kernel.
 constexpr int64_t kGemmMaxM = 1 << 20;
 
@@ -2032,10 +2038,11 @@ int w4a16_dequantize_f16(const uint8_t* packed_weights, const void* scales, void
     const int64_t words = chunks * 4;   // 32-bit words of codes, 8 weights each
     const int64_t blocks = (words + 1023) / 1024;
     if (blocks > INT32_MAX) return fail(W4A16_ERR_TOO_LARGE, "too many chunks for one launch");
-    hipLaunchKernelGGL(w4a16::dequantize_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), packed_weights, static_cast<const w4a16::f16*>(scales),
-                       static_cast<w4a16::f16*>(output), words, (int)(K / 8), (int)(group_size / 8),
-                       (int)(K / group_size));
+    const int wpg = (int)(group_size / 8);
+    const int shift = (wpg & (wpg - 1)) == 0 ? __builtin_ctz((unsigned)wpg) : -1;
+    const auto kern = N * K * 2 > kDequantStreamBytes ? w4a16::dequantize_kernel<true> : w4a16::dequantize_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream), packed_weights,
+                       static_cast<const w4a16::f16*>(scales), static_cast<w4a16::f16*>(output), words, wpg, shift);
     return check_launch();
 }
 

@@ -1178,41 +1178,44 @@ linear_generic(const f16* __restrict__ x, const uint8_t* __restrict__ w,
 // operands rounds the exact product once (round to nearest even, subnormals
 // kept), which is the value of reference w4a16/reference.py:38-46 followed by
 // .to(torch.float16).
+// K is a multiple of G, so groups lie end to end over the whole matrix: a
+// word's scale is its index over the words of a group (wpg; shift = its
+// logarithm where it is a power of two, else -1), whatever its row. Bound:
+// the store stream. 28672 x 8192 (591 MB): 100 us, 5.9 TB/s (a copy reaches
+// 5.1); 132 us with each word's row found by 64-bit division and its scale
+// requested only when its weights had arrived.
 // ---------------------------------------------------------------------------
+template <bool STREAM>
 __global__ void __launch_bounds__(256)
 dequantize_kernel(const uint8_t* __restrict__ w, const f16* __restrict__ scales,
-                  f16* __restrict__ out, int64_t words, int words_per_row,
-                  int words_per_group, int groups_per_row) {
+                  f16* __restrict__ out, int64_t words, int wpg, int shift) {
     const int lane = threadIdx.x & 63;
     const int64_t base = ((int64_t)blockIdx.x * 256 + (threadIdx.x & ~63)) * 4;   // the wavefront's first word
     const uint32_t* wp = reinterpret_cast<const uint32_t*>(w);
     uint32_t d[4];
+    f16 s[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) d[q] = __builtin_nontemporal_load(wp + min(base + 64 * q + lane, words - 1));
+    const int64_t g0 = shift >= 0 ? base >> shift : base / wpg;   // uniform
+    const uint32_t r0 = (uint32_t)(base - g0 * wpg);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int64_t j = base + 64 * q + lane;
-        d[q] = j < words ? __builtin_nontemporal_load(wp + j) : 0u;
+        const uint32_t r = r0 + (uint32_t)min((int64_t)(64 * q + lane), words - 1 - base);
+        s[q] = scales[g0 + (shift >= 0 ? r >> shift : r / (uint32_t)wpg)];
     }
-    // row and word-in-row of word base + lane, then steps of 64 words
-    int64_t n = (base + lane) / words_per_row;
-    int c = (int)(base + lane - n * words_per_row);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const int64_t j = base + 64 * q + lane;
         if (j < words) {
-            const f16 s = scales[n * groups_per_row + c / words_per_group];
-            const f16x2 ss = {s, s};
+            const f16x2 ss = {s[q], s[q]};
             const uint32_t u = d[q] ^ 0x88888888u;
             u32x4 v;
             v.x = as_u32(unpack_byte_pair<0>(u) * ss);
             v.y = as_u32(unpack_byte_pair<1>(u) * ss);
             v.z = as_u32(unpack_byte_pair<2>(u) * ss);
             v.w = as_u32(unpack_byte_pair<3>(u) * ss);
-            reinterpret_cast<u32x4*>(out)[j] = v;
-        }
-        c += 64;
-        while (c >= words_per_row) {   // 64 words may cross several short rows
-            c -= words_per_row;
-            ++n;
+            if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(out) + j);
+            else reinterpret_cast<u32x4*>(out)[j] = v;
         }
     }
 }
