@@ -1191,6 +1191,7 @@ dequantize_kernel(const uint8_t* __restrict__ w, const f16* __restrict__ scales,
                   f16* __restrict__ out, int64_t words, int wpg, int shift) {
     const int lane = threadIdx.x & 63;
     const int64_t base = ((int64_t)blockIdx.x * 256 + (threadIdx.x & ~63)) * 4;   // the wavefront's first word
+    if (base >= words) return;   // a wavefront past the end: the clamps below need one word of its own
     const uint32_t* wp = reinterpret_cast<const uint32_t*>(w);
     uint32_t d[4];
     f16 s[4];

@@ -7,7 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from _cases import assert_parity, expected, make_case
+from tests._cases import assert_parity, expected, make_case
 from nibble_amd import _lib
 
 pytestmark = pytest.mark.gpu

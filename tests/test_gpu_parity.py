@@ -795,3 +795,18 @@ def test_dequantize_all_codes_all_finite_scales(gpu):
     # NaN payloads are not part of the contract; scales here are finite, so
     # 0 * finite never makes NaN
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("group", [32, 96, 128, 512])
+@pytest.mark.parametrize("n,groups", [(1, 1), (3, 1), (8, 1), (5, 7), (33, 9)])
+def test_dequantize_small_and_ragged(gpu, group, n, groups):
+    """Fewer words than a workgroup's, last wavefronts with part of their words
+    or none, and groups that are no power of two: every fp16 bit."""
+    gen = torch.Generator().manual_seed(n * groups + group)
+    p = torch.randint(0, 256, (n, groups * group // 2), generator=gen, dtype=torch.uint8)
+    s = (torch.rand((n, groups), generator=gen) + 0.01).to(torch.float16)
+    print(f"[case] dequantize N={n} K={groups * group} G={group}", flush=True)
+    out = torch.ops.w4a16.dequantize(p.to(gpu), s.to(gpu), group)
+    torch.cuda.synchronize()
+    ref = torch.from_numpy(oracle.dequantize_f16(p.numpy(), s.numpy(), group))
+    assert torch.equal(out.cpu().view(torch.int16), ref.view(torch.int16))
