@@ -65,7 +65,8 @@ def linear_cuda(
     gfx950 kernels; anything else runs the generic HIP kernel.
     """
     _require_extension()
-    return torch.ops.w4a16.linear(activations, packed_weights, scales, group_size)
+    # the overload itself: naming the packet looks it up on every call (about 1 us)
+    return torch.ops.w4a16.linear.default(activations, packed_weights, scales, group_size)
 
 
 def dequantize_cuda(

@@ -159,32 +159,33 @@ class QuantizedLinear(torch.nn.Module):
             raise TypeError("activations must have dtype torch.float16")
         if activations.requires_grad:
             raise RuntimeError("activations must not require grad")
-        if activations.device != self.packed_weights.device:
+        packed, scales = self.packed_weights, self.scales   # buffers: each look-up costs about 0.3 us
+        if activations.device != packed.device:
             raise ValueError("activations and packed_weights must share a device")
 
-        output_shape = (*activations.shape[:-1], self.out_features)
         # The kernels need a dense [M, K] matrix; views from attention reshapes are copied.
-        flat = activations.contiguous().reshape(-1, self.in_features)
+        matrix = activations.ndim == 2
+        flat = activations.contiguous() if matrix else activations.contiguous().reshape(-1, self.in_features)
         rows = flat.shape[0]
         if flat.is_cuda:
-            if not self.packed_weights.is_contiguous():
+            if not packed.is_contiguous():
                 raise ValueError("packed_weights must be contiguous")
-            if not self.scales.is_contiguous():
+            if not scales.is_contiguous():
                 raise ValueError("scales must be contiguous")
             if self.fused and rows <= FUSED_MAX_ROWS:
-                out = linear_cuda(flat, self.packed_weights, self.scales, self.group_size)
+                out = linear_cuda(flat, packed, scales, self.group_size)
             elif self.fused and self.group_size == 128 and rows <= self._native_rows():
-                out = linear_cuda(flat, self.packed_weights, self.scales, self.group_size)
+                out = linear_cuda(flat, packed, scales, self.group_size)
             elif self.group_size % 32 == 0:
                 out = self._dequant_linear(flat)
             else:
-                out = linear_cuda(flat, self.packed_weights, self.scales, self.group_size)
+                out = linear_cuda(flat, packed, scales, self.group_size)
         else:
-            out = linear_reference(flat, self.packed_weights, self.scales, self.group_size)
-        out = out.reshape(output_shape)
-        if self.bias is not None:
-            out = out + self.bias
-        return out
+            out = linear_reference(flat, packed, scales, self.group_size)
+        if not matrix:
+            out = out.reshape(*activations.shape[:-1], self.out_features)
+        bias = self.bias
+        return out if bias is None else out + bias
 
 
 # The name the W4A16 API documentation uses for the same class.
