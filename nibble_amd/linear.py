@@ -136,11 +136,21 @@ class QuantizedLinear(torch.nn.Module):
             f"group_size={self.group_size}, bias={self.bias is not None}, fused={self.fused}"
         )
 
-    def _native_rows(self) -> int:
-        """Most prompt rows that take the W4A16 GEMM: ``native_max_rows``, twice
-        its default on small layers (a value set by the caller stands as it is)."""
-        small = self.in_features * self.out_features <= NATIVE_GEMM_SMALL_LAYER
-        return self.native_max_rows * (2 if small and self.native_max_rows == NATIVE_GEMM_MAX_ROWS else 1)
+    def _takes_gemm(self, flat: torch.Tensor) -> bool:
+        """Whether these prompt rows take the W4A16 GEMM: up to ``native_max_rows``,
+        and up to twice its default on small layers (a value other than the
+        default stands as it is). Past ``native_max_rows`` only rows that start
+        on 16 bytes, which the GEMM needs: the library's scalar kernel, which
+        takes the others, is far behind the dense GEMM there."""
+        rows = flat.shape[0]
+        if rows <= self.native_max_rows:
+            return True
+        return (
+            self.native_max_rows == NATIVE_GEMM_MAX_ROWS
+            and rows <= 2 * NATIVE_GEMM_MAX_ROWS
+            and self.in_features * self.out_features <= NATIVE_GEMM_SMALL_LAYER
+            and flat.storage_offset() % 8 == 0
+        )
 
     def _dequant_linear(self, activations: torch.Tensor) -> torch.Tensor:
         """fp16 weight matrix from the packed codes, then a dense GEMM."""
@@ -174,7 +184,7 @@ class QuantizedLinear(torch.nn.Module):
                 raise ValueError("scales must be contiguous")
             if self.fused and rows <= FUSED_MAX_ROWS:
                 out = linear_cuda(flat, packed, scales, self.group_size)
-            elif self.fused and self.group_size == 128 and rows <= self._native_rows():
+            elif self.fused and self.group_size == 128 and self._takes_gemm(flat):
                 out = linear_cuda(flat, packed, scales, self.group_size)
             elif self.group_size % 32 == 0:
                 out = self._dequant_linear(flat)

@@ -1,0 +1,65 @@
+"""Prompt rows (M > 16) where the library chooses the GEMM shape by estimated
+time, and the rows past which QuantizedLinear hands over to the dense GEMM."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from nibble_amd.cuda import dequantize_cuda
+from nibble_amd.linear import NATIVE_GEMM_MAX_ROWS, QuantizedLinear
+from tests._cases import make_case
+
+
+# a row past a tile of 16, 32, 64 and 128, and past a second round of tiles;
+# K from the least that is chosen by time, and group counts that no K split
+# divides (9, 11, 13); N below one tile, ragged, and an even number of tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [17, 24, 32, 33, 65, 127, 200, 385, 513, 700, 1024])
+@pytest.mark.parametrize("k,n", [(1024, 24), (1152, 515), (1408, 4100), (1664, 1000), (2048, 5632), (5632, 2049)])
+def test_prompt_rows_by_estimated_time(gpu, m, k, n):
+    """The op against 64-bit sums over the dequantized weights: half an ulp of
+    the fp16 output, and for the fp32 sums 2^-23 of the sum of magnitudes for
+    each of the K / 16 + 32 additions that one output passes through at most."""
+    x, p, s = (t.to(gpu) for t in make_case(m, k, n, seed=m + k + n))
+    print(f"[case] M={m} K={k} N={n}", flush=True)
+    out = torch.ops.w4a16.linear(x, p, s, 128)
+    torch.cuda.synchronize()
+    wt = dequantize_cuda(p, s, 128).double().t().contiguous()
+    ref, size = x.double() @ wt, x.double().abs() @ wt.abs()
+    bound = ref.abs() * 2 ** -11 + (k / 16 + 32) * 2 ** -23 * size + 2 ** -25
+    err = (out.double() - ref).abs()
+    assert torch.all(err <= bound), f"worst {float((err / bound).max()):.3f} of the bound"
+
+
+def _layer(n, k):
+    return QuantizedLinear(torch.zeros((n, k // 2), dtype=torch.uint8), torch.ones((n, k // 128), dtype=torch.float16))
+
+
+def test_rows_that_take_the_gemm():
+    top = NATIVE_GEMM_MAX_ROWS
+    rows = torch.zeros((2 * top + 2, 256), dtype=torch.float16)
+    small = _layer(8, 256)
+    assert [small._takes_gemm(rows[:m]) for m in (top, top + 1, 2 * top, 2 * top + 1)] == [True, True, True, False]
+    shifted = rows.reshape(-1)[1:1 + (top + 1) * 256].view(top + 1, 256)   # contiguous, 2 bytes past the alignment
+    assert not small._takes_gemm(shifted) and small._takes_gemm(shifted[:top])
+    small.native_max_rows = 100
+    assert small._takes_gemm(rows[:100]) and not small._takes_gemm(rows[:101])
+    large = _layer(96000, 256)   # 24.6M weights
+    assert large._takes_gemm(rows[:top]) and not large._takes_gemm(rows[:top + 1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [513, 1024, 1025])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_module_rows_past_the_gemm(gpu, rows, shift):
+    k, n = 1024, 520
+    x, p, s = (t.to(gpu) for t in make_case(rows, k, n, seed=rows))
+    store = torch.empty((rows * k + 1,), dtype=torch.float16, device=gpu)
+    store[shift:shift + rows * k] = x.reshape(-1)
+    view = store[shift:shift + rows * k].view(rows, k)
+    print(f"[case] rows={rows} shift={shift}", flush=True)
+    out = QuantizedLinear(p, s, group_size=128)(view)
+    ref = x.double() @ dequantize_cuda(p, s, 128).double().t().contiguous()
+    # the bound of the other module tests on dequantized weights
+    torch.testing.assert_close(out.double(), ref, rtol=1e-3, atol=1e-3)
