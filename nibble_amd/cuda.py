@@ -53,6 +53,20 @@ def _require_extension() -> None:
         ) from _EXTENSION_LOAD_ERROR
 
 
+def addressable(tensor: torch.Tensor) -> bool:
+    """Whether a choice may look at where this tensor's memory starts: an
+    ordinary tensor of a call that runs now. False for a traced call (its
+    graph also serves other tensors), under a dispatch mode, for a wrapper of
+    ``torch.func`` and for a subclass, which may have no memory of their own."""
+    return (
+        not torch.compiler.is_compiling()
+        and type(tensor) in (torch.Tensor, torch.nn.Parameter)
+        and not torch.jit.is_tracing()
+        and torch._C._len_torch_dispatch_stack() == 0
+        and not torch._C._functorch.is_functorch_wrapped_tensor(tensor)
+    )
+
+
 def linear_cuda(
     activations: torch.Tensor,
     packed_weights: torch.Tensor,

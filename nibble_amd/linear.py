@@ -29,7 +29,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
-from nibble_amd.cuda import dequantize_cuda, linear_cuda
+from nibble_amd.cuda import addressable, dequantize_cuda, linear_cuda
 from nibble_amd.quantization import quantize_and_pack_weights
 from nibble_amd.reference import dequantize_weights, linear_reference
 
@@ -141,7 +141,9 @@ class QuantizedLinear(torch.nn.Module):
         and up to twice its default on small layers (a value other than the
         default stands as it is). Past ``native_max_rows`` only rows that start
         on 16 bytes, which the GEMM needs: the library's scalar kernel, which
-        takes the others, is far behind the dense GEMM there."""
+        takes the others, is far behind the dense GEMM there. Where the tensor
+        has no address to test (torch.compile and the like) these rows keep
+        dequantize + the dense GEMM."""
         rows = flat.shape[0]
         if rows <= self.native_max_rows:
             return True
@@ -149,6 +151,7 @@ class QuantizedLinear(torch.nn.Module):
             self.native_max_rows == NATIVE_GEMM_MAX_ROWS
             and rows <= 2 * NATIVE_GEMM_MAX_ROWS
             and self.in_features * self.out_features <= NATIVE_GEMM_SMALL_LAYER
+            and addressable(flat)
             and flat.storage_offset() % 8 == 0
         )
 

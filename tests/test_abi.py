@@ -688,3 +688,31 @@ def test_workspace_plan_ring_slices(m, k, n, sk, sn, depth, slices):
     assert plan == {"kernel": "pair_ring", "rows": sn, "splits": sk, "unroll": depth, "max_blocks": slices}
     plain = _lib.plan_linear(ALIGNED, ALIGNED, m, n, k, 128)
     assert not (plain["kernel"] == "pair_ring" and plain["max_blocks"] > 1)
+
+
+@pytest.mark.parametrize("rows", [4, 512, 513, 600, 1024, 1025])
+def test_module_traces_whole(rows):
+    """torch.compile(fullgraph=True) of a small layer over GPU tensors without
+    data: rows where an eager call looks at its operands' addresses (513..1024)
+    trace like the others, and take dequantize + the dense GEMM."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from nibble_amd.linear import QuantizedLinear
+
+    graphs = []
+
+    def backend(gm, _):
+        graphs.append([str(node.target) for node in gm.graph.nodes])
+        return gm
+
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        layer = QuantizedLinear(torch.zeros((64, 128), dtype=torch.uint8, device="cuda"),
+                                torch.ones((64, 2), dtype=torch.float16, device="cuda"))
+        x = torch.zeros((rows, 256), dtype=torch.float16, device="cuda")
+        torch._dynamo.reset()
+        out = torch.compile(layer, fullgraph=True, backend=backend)(x)
+        assert tuple(out.shape) == (rows, 64)
+        assert tuple(layer(x).shape) == (rows, 64)
+    assert len(graphs) == 1
+    assert any("w4a16.linear" in target for target in graphs[0]) == (rows <= 512)
+    assert any("w4a16.dequantize" in target for target in graphs[0]) == (rows > 512)

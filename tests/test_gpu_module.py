@@ -196,7 +196,7 @@ def test_load_packed_state_dict_does_not_materialize_fp16(gpu):
     assert src.packed_weights.numel() + src.scales.numel() * 2 <= delta < k * n * 2
 
 
-@pytest.mark.parametrize("rows", [1, 4, 24])
+@pytest.mark.parametrize("rows", [1, 4, 24, 600, 1024])
 def test_traces_under_torch_compile(gpu, rows):
     torch.manual_seed(0)
     p, s = quantize_and_pack_weights(torch.randn((256, 512), dtype=torch.float16, device=gpu), 128)
