@@ -139,10 +139,10 @@ class QuantizedLinear(torch.nn.Module):
     def _takes_gemm(self, flat: torch.Tensor) -> bool:
         """Whether these prompt rows take the W4A16 GEMM: up to ``native_max_rows``,
         and up to twice its default on small layers (a value other than the
-        default stands as it is). Past ``native_max_rows`` only rows that start
-        on 16 bytes, which the GEMM needs: the library's scalar kernel, which
-        takes the others, is far behind the dense GEMM there. Where the tensor
-        has no address to test (torch.compile and the like) these rows keep
+        default stands as it is). Past ``native_max_rows`` only rows and weights
+        that start on 16 bytes, which the GEMM needs: the library's scalar
+        kernel, which takes the others, is far behind the dense GEMM there, and
+        dequantize refuses such weights. Where a tensor has no address to test (torch.compile and the like) these rows keep
         dequantize + the dense GEMM."""
         rows = flat.shape[0]
         if rows <= self.native_max_rows:
@@ -151,8 +151,7 @@ class QuantizedLinear(torch.nn.Module):
             self.native_max_rows == NATIVE_GEMM_MAX_ROWS
             and rows <= 2 * NATIVE_GEMM_MAX_ROWS
             and self.in_features * self.out_features <= NATIVE_GEMM_SMALL_LAYER
-            and addressable(flat)
-            and flat.storage_offset() % 8 == 0
+            and all(addressable(t) and t.data_ptr() % 16 == 0 for t in (flat, self.packed_weights))
         )
 
     def _dequant_linear(self, activations: torch.Tensor) -> torch.Tensor:

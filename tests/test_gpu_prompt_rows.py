@@ -49,6 +49,41 @@ def test_rows_that_take_the_gemm():
     assert large._takes_gemm(rows[:top]) and not large._takes_gemm(rows[:top + 1])
 
 
+def _past_alignment(dtype, shape, shift):
+    """A tensor whose own storage starts `shift` bytes past 16, at storage offset 0."""
+    size = torch.zeros(shape, dtype=dtype).nbytes
+    buffer = bytearray(size + 32)
+    start = -torch.frombuffer(buffer, dtype=torch.uint8).data_ptr() % 16 + shift
+    out = torch.frombuffer(buffer, dtype=dtype, offset=start, count=size // dtype.itemsize).view(shape)
+    assert out.data_ptr() % 16 == shift and out.storage_offset() == 0
+    return out
+
+
+def test_rows_that_take_the_gemm_start_on_16_bytes():
+    """The address decides, not the offset within a storage that may itself start anywhere."""
+    rows = NATIVE_GEMM_MAX_ROWS + 1
+    layer = _layer(8, 256)
+    for shift in range(0, 16, 2):
+        assert layer._takes_gemm(_past_alignment(torch.float16, (rows, 256), shift)) == (shift == 0)
+    store = _past_alignment(torch.float16, (rows * 256 + 1,), 14)   # one element on: 16-byte aligned
+    assert layer._takes_gemm(store[1:].view(rows, 256))
+    odd = QuantizedLinear(_past_alignment(torch.uint8, (8, 128), 4), torch.ones((8, 2), dtype=torch.float16))
+    assert odd._takes_gemm(torch.zeros((rows - 1, 256), dtype=torch.float16))
+    assert not odd._takes_gemm(torch.zeros((rows, 256), dtype=torch.float16))
+
+
+@pytest.mark.gpu
+def test_module_refuses_misaligned_weights_past_the_gemm(gpu):
+    """dequantize refuses weights that do not start on 16 bytes; the module does at these rows, too."""
+    _, p, s = make_case(1, 256, 8, seed=0)
+    store = torch.empty((p.numel() + 4,), dtype=torch.uint8, device=gpu)
+    store[4:] = p.reshape(-1).to(gpu)
+    layer = QuantizedLinear(store[4:].view_as(p), s.to(gpu))
+    for rows in (513, 1024, 1025):
+        with pytest.raises(RuntimeError, match="16-byte aligned"):
+            layer(torch.zeros((rows, 256), dtype=torch.float16, device=gpu))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows", [513, 1024, 1025])
 @pytest.mark.parametrize("shift", [0, 1])
