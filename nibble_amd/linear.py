@@ -93,8 +93,9 @@ class QuantizedLinear(torch.nn.Module):
         self.fused = fused
         # prompt rows up to this count take the W4A16 GEMM when fused (set it
         # to FUSED_MAX_ROWS for the reference's routing: dequantize + GEMM for
-        # every M > 8)
-        self.native_max_rows = NATIVE_GEMM_MAX_ROWS
+        # every M > 8; a value that is set stands as it is, whatever the layer)
+        small = self.in_features * self.out_features <= NATIVE_GEMM_SMALL_LAYER
+        self.native_max_rows = 2 * NATIVE_GEMM_MAX_ROWS if small else NATIVE_GEMM_MAX_ROWS
 
     @classmethod
     def from_float(cls, layer: torch.nn.Linear, group_size: int = 128, fused: bool = True) -> "QuantizedLinear":
@@ -137,22 +138,16 @@ class QuantizedLinear(torch.nn.Module):
         )
 
     def _takes_gemm(self, flat: torch.Tensor) -> bool:
-        """Whether these prompt rows take the W4A16 GEMM: up to ``native_max_rows``,
-        and up to twice its default on small layers (a value other than the
-        default stands as it is). Past ``native_max_rows`` only rows and weights
-        that start on 16 bytes, which the GEMM needs: the library's scalar
-        kernel, which takes the others, is far behind the dense GEMM there, and
-        dequantize refuses such weights. Where a tensor has no address to test (torch.compile and the like) these rows keep
-        dequantize + the dense GEMM."""
+        """Whether these prompt rows take the W4A16 GEMM: up to ``native_max_rows``.
+        Past NATIVE_GEMM_MAX_ROWS only rows and weights that start on 16 bytes,
+        which the GEMM needs: the library's scalar kernel, which takes the
+        others, is far behind the dense GEMM there, and dequantize refuses such
+        weights. Where a tensor has no address to test (torch.compile and the
+        like) these rows keep dequantize + the dense GEMM."""
         rows = flat.shape[0]
-        if rows <= self.native_max_rows:
-            return True
-        return (
-            self.native_max_rows == NATIVE_GEMM_MAX_ROWS
-            and rows <= 2 * NATIVE_GEMM_MAX_ROWS
-            and self.in_features * self.out_features <= NATIVE_GEMM_SMALL_LAYER
-            and all(addressable(t) and t.data_ptr() % 16 == 0 for t in (flat, self.packed_weights))
-        )
+        if rows > self.native_max_rows or rows <= NATIVE_GEMM_MAX_ROWS:
+            return rows <= self.native_max_rows
+        return all(addressable(t) and t.data_ptr() % 16 == 0 for t in (flat, self.packed_weights))
 
     def _dequant_linear(self, activations: torch.Tensor) -> torch.Tensor:
         """fp16 weight matrix from the packed codes, then a dense GEMM."""

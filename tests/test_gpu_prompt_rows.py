@@ -49,6 +49,17 @@ def test_rows_that_take_the_gemm():
     assert large._takes_gemm(rows[:top]) and not large._takes_gemm(rows[:top + 1])
 
 
+def test_rows_that_a_caller_sets_stand():
+    """512 set by a caller is no more than 512, on a small layer, too; a larger value counts on a large one."""
+    top = NATIVE_GEMM_MAX_ROWS
+    rows = torch.zeros((2 * top + 2, 256), dtype=torch.float16)
+    small, large = _layer(8, 256), _layer(96000, 256)
+    small.native_max_rows = top
+    assert small._takes_gemm(rows[:top]) and not small._takes_gemm(rows[:top + 1])
+    large.native_max_rows = 2 * top + 1
+    assert large._takes_gemm(rows[:2 * top + 1]) and not large._takes_gemm(rows)
+
+
 def _past_alignment(dtype, shape, shift):
     """A tensor whose own storage starts `shift` bytes past 16, at storage offset 0."""
     size = torch.zeros(shape, dtype=dtype).nbytes
