@@ -44,12 +44,26 @@ FUSED_MAX_ROWS = 8
 # 131 us, 2048 x 11264 75 against 69) and on most layers at M = 2048, so
 # longer prompts keep it.
 NATIVE_GEMM_MAX_ROWS = 512
-# Layers of at most this many weights keep the W4A16 GEMM up to twice those
-# rows: 2048 x 5632 at M = 600 22.9 against 35.6 us, 5632 x 2048 at M = 1024
-# 35.4 against 46.9, 2048 x 11264 at M = 1024 61.0 against 69.4; larger layers
-# lose some (4096 x 14336 at M = 600 104.8 against 96.8, 4096 x 6144 at M = 768
-# 63.2 against 60.9).
-NATIVE_GEMM_SMALL_LAYER = 24_000_000
+
+
+def gemm_max_rows(n: int, k: int) -> int:
+    """Rows up to which the W4A16 GEMM of a layer keeps up with dequantize + the
+    dense GEMM: a sweep of 513..1024 rows over layers of up to 24M weights
+    (graph timing, rotated weights), in which it loses no more than 1.5%
+    anywhere below these lines. Its tiles fill whole rounds of the 256 CUs on
+    small and narrow layers (K x N at 1024 rows, us: 5632 x 2048 36.6 against
+    45.3, 14336 x 1024 57.7 against 61.9, 2048 x 4096 26.6 against 34.8).
+    Others start a second round past 704 rows (4096 x 5632 at 704 50.6 against
+    54.0, at 705 62.8 against 55.0; 1408 x 16384 at 704 45.6 against 50.5, at
+    1024 64.9 against 58.2), the widest at once (1024 x 20480 at 576 49.1
+    against 43.5). Rows shorter than 1024 weights run shapes chosen by their
+    grid alone, which lose here and there past 512 outputs (128 x 1024 at 576
+    12.1 against 8.2)."""
+    if n * k > 24_000_000 or (k < 1024 and n > 512):
+        return NATIVE_GEMM_MAX_ROWS
+    if n <= 2048 or n * k <= (12_000_000 if n <= 4096 else 9_000_000):
+        return 2 * NATIVE_GEMM_MAX_ROWS
+    return 704 if n <= 5632 or (n <= 16384 and k <= 2048) else NATIVE_GEMM_MAX_ROWS
 
 
 class QuantizedLinear(torch.nn.Module):
@@ -94,8 +108,7 @@ class QuantizedLinear(torch.nn.Module):
         # prompt rows up to this count take the W4A16 GEMM when fused (set it
         # to FUSED_MAX_ROWS for the reference's routing: dequantize + GEMM for
         # every M > 8; a value that is set stands as it is, whatever the layer)
-        small = self.in_features * self.out_features <= NATIVE_GEMM_SMALL_LAYER
-        self.native_max_rows = 2 * NATIVE_GEMM_MAX_ROWS if small else NATIVE_GEMM_MAX_ROWS
+        self.native_max_rows = gemm_max_rows(self.out_features, self.in_features)
 
     @classmethod
     def from_float(cls, layer: torch.nn.Linear, group_size: int = 128, fused: bool = True) -> "QuantizedLinear":

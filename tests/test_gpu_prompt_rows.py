@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from nibble_amd.cuda import dequantize_cuda
-from nibble_amd.linear import NATIVE_GEMM_MAX_ROWS, QuantizedLinear
+from nibble_amd.linear import NATIVE_GEMM_MAX_ROWS, QuantizedLinear, gemm_max_rows
 from tests._cases import make_case
 
 
@@ -47,6 +47,16 @@ def test_rows_that_take_the_gemm():
     assert small._takes_gemm(rows[:100]) and not small._takes_gemm(rows[:101])
     large = _layer(96000, 256)   # 24.6M weights
     assert large._takes_gemm(rows[:top]) and not large._takes_gemm(rows[:top + 1])
+
+
+@pytest.mark.parametrize("k,n,rows", [
+    (2048, 2048, 1024), (5632, 2048, 1024), (11008, 2048, 1024), (14336, 1536, 1024), (2048, 4096, 1024),
+    (1024, 8192, 1024), (128, 512, 1024),                                         # faster up to 1024 rows
+    (4096, 2560, 1024), (5632, 2560, 704), (8192, 2560, 704), (4096, 4096, 704), (2048, 5632, 704),
+    (4096, 5632, 704), (2048, 11264, 704), (1408, 16384, 704), (1024, 16384, 704),   # slower past 704
+    (1024, 20480, 512), (2816, 8192, 512), (128, 1024, 512), (512, 16384, 512), (4096, 6144, 512)])
+def test_rows_up_to_which_the_gemm_keeps_up(k, n, rows):
+    assert gemm_max_rows(n, k) == rows
 
 
 def test_rows_that_a_caller_sets_stand():
