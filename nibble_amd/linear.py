@@ -173,7 +173,8 @@ class QuantizedLinear(torch.nn.Module):
     def forward(self, activations: torch.Tensor) -> torch.Tensor:
         if activations.ndim < 1:
             raise ValueError("activations must have at least one dimension")
-        if activations.shape[-1] != self.in_features:
+        in_features = self.in_features
+        if activations.shape[-1] != in_features:
             raise ValueError("activations last dimension must equal in_features")
         if activations.dtype != torch.float16:
             raise TypeError("activations must have dtype torch.float16")
@@ -184,8 +185,9 @@ class QuantizedLinear(torch.nn.Module):
             raise ValueError("activations and packed_weights must share a device")
 
         # The kernels need a dense [M, K] matrix; views from attention reshapes are copied.
-        matrix = activations.ndim == 2
-        flat = activations.contiguous() if matrix else activations.contiguous().reshape(-1, self.in_features)
+        # Rows of no features have no row count to infer, and the reshape refuses them.
+        matrix = activations.ndim == 2 and in_features > 0
+        flat = activations.contiguous() if matrix else activations.contiguous().reshape(-1, in_features)
         rows = flat.shape[0]
         if flat.is_cuda:
             if not packed.is_contiguous():

@@ -299,3 +299,10 @@ def test_tiny_hf_llama_round_trip():
     assert not any(isinstance(m, torch.nn.Linear) for m in target.modules() if m is not target)
     assert torch.equal(source.model.rotary_emb.inv_freq, target.model.rotary_emb.inv_freq)
     assert torch.equal(result, expected)
+
+
+@pytest.mark.parametrize("shape", [(0,), (2, 0), (2, 3, 0)])
+def test_rows_of_no_features_are_refused(shape):
+    layer = QuantizedLinear(torch.zeros((4, 0), dtype=torch.uint8), torch.zeros((4, 0), dtype=torch.float16))
+    with pytest.raises(RuntimeError):
+        layer(torch.zeros(shape, dtype=torch.float16))
