@@ -18,7 +18,7 @@ from __future__ import annotations
 import torch
 from torch.autograd import forward_ad
 
-from nibble_amd.cuda import cuda_extension_available, quantize_cuda
+from nibble_amd.cuda import addressable, cuda_extension_available, quantize_cuda
 
 
 def pack_int4(quantized_weights: torch.Tensor) -> torch.Tensor:
@@ -105,13 +105,13 @@ def _native(weights: torch.Tensor, group_size: int) -> bool:
     """Whether the HIP quantizer takes these weights: a GPU matrix of the types
     the quantizer accepts, groups of a power of two from 16 to 512 (lanes of
     one wavefront), 16-byte aligned once contiguous. Everything else, and
-    every call that the checks of the torch ops reject, that is traced or that
-    asks for derivatives, keeps the torch ops."""
+    every call that the checks of the torch ops reject, that is traced, runs
+    under a ``torch.func`` transform or asks for derivatives, keeps the torch
+    ops."""
     return (
-        type(weights) in (torch.Tensor, torch.nn.Parameter)
+        addressable(weights)
         and weights.is_cuda
         and cuda_extension_available()
-        and not torch.compiler.is_compiling()
         and weights.dtype in (torch.float16, torch.float32)
         and weights.ndim == 2
         and weights.numel() > 0

@@ -306,3 +306,46 @@ def test_rows_of_no_features_are_refused(shape):
     layer = QuantizedLinear(torch.zeros((4, 0), dtype=torch.uint8), torch.zeros((4, 0), dtype=torch.float16))
     with pytest.raises(RuntimeError):
         layer(torch.zeros(shape, dtype=torch.float16))
+
+
+def _quantizer_calls():
+    """Traced and transformed calls of the quantizer, which keep its torch ops."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    def scales(w):
+        return quantize_and_pack_weights(w, 128)[1].float()
+
+    def dual(w):
+        with forward_ad.dual_level():
+            return forward_ad.unpack_dual(scales(forward_ad.make_dual(w, torch.ones_like(w)))).tangent
+
+    def mode(w):
+        with Seen():
+            return scales(w)
+
+    return {
+        "jvp": lambda w: torch.func.jvp(scales, (w,), (torch.ones_like(w),))[1],
+        "grad": lambda w: torch.func.grad(lambda v: scales(v).sum())(w),
+        "functionalize": lambda w: torch.func.functionalize(scales)(w),
+        "jit.trace": lambda w: torch.jit.trace(scales, (w,), check_trace=False)(w),
+        "dual": dual,
+        "mode": mode,
+        "grad mode": lambda w: torch.autograd.grad(scales(w.requires_grad_()).sum(), w)[0],
+    }
+
+
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("name", list(_quantizer_calls()))
+def test_quantizer_traced_or_transformed(name, monkeypatch):
+    """These calls give on a GPU tensor what they give on a CPU one: with
+    is_cuda answering True, any that took the native op would find no CPU
+    kernel for it, or no data pointer to look at."""
+    w = torch.randn((4, 256), generator=torch.Generator().manual_seed(3))
+    expected = _quantizer_calls()[name](w.clone())
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    assert torch.equal(_quantizer_calls()[name](w.clone()), expected)
