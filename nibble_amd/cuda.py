@@ -1,4 +1,5 @@
-"""Python wrappers of the torch ops ``w4a16::linear`` / ``w4a16::dequantize``.
+"""Python wrappers of the torch ops ``w4a16::linear``, ``w4a16::dequantize`` and
+``w4a16::quantize``.
 
 Mirrors reference ``w4a16/cuda.py``: importing the compiled extension
 (``nibble_amd._C``, here a thin libtorch shim over the HIP C ABI) registers
@@ -33,6 +34,14 @@ if _EXTENSION_LOAD_ERROR is None:
     def _dequantize_fake(packed_weights, scales, group_size):
         return packed_weights.new_empty(
             (packed_weights.shape[0], packed_weights.shape[1] * 2), dtype=torch.float16
+        )
+
+    @torch.library.register_fake("w4a16::quantize")
+    def _quantize_fake(weights, group_size):
+        rows, cols = weights.shape
+        return (
+            weights.new_empty((rows, cols // 2), dtype=torch.uint8),
+            weights.new_empty((rows, cols // group_size), dtype=torch.float16),
         )
 
 

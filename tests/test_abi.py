@@ -656,6 +656,18 @@ def test_fake_kernels_give_shapes():
     assert tuple(w.shape) == (8, 256) and w.dtype == torch.float16
 
 
+def test_fake_quantize_gives_shapes():
+    import nibble_amd  # noqa: F401
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode():
+        for dtype in (torch.float16, torch.float32):
+            w = torch.empty((6, 384), dtype=dtype, device="cuda")
+            packed, scales = torch.ops.w4a16.quantize(w, 64)
+            assert tuple(packed.shape) == (6, 192) and packed.dtype == torch.uint8 and packed.device == w.device
+            assert tuple(scales.shape) == (6, 6) and scales.dtype == torch.float16 and scales.device == w.device
+
+
 def test_split_plans_are_launchable():
     """Every split-K plan the router can make (M = 3..8, K = 16512..65536 and
     beyond) is one the launcher accepts: 2..16 slices, none empty, a slice's
