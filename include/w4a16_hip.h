@@ -274,12 +274,13 @@ int w4a16_plan_linear_ws(const void* activations, const uint8_t* packed_weights,
  *     W4A16_KERNEL_GEMM_LDS with 32-row tiles; (rows, max_blocks, unroll,
  *     splits) one of (4, 2, 4, 1), (4, 1, 4, 1), (2, 1, 4, 2), (2, 2, 2, 2),
  *     (2, 2, 4, 1), (4, 1, 2, 2), (2, 1, 2, 4), (2, 1, 1, 4).
- *   W4A16_KERNEL_GENERIC: the scalar kernel, other arguments ignored, unless
- *     max_blocks = 1 and group_size is 32 or 64, M <= 8, K a multiple of 128,
- *     activations and weights 16-byte and scales 256 / group_size-byte
- *     aligned: then its matrix-core form, splits = wavefronts splitting K
- *     (1|2|4|8), rows = wavefronts on 8-row blocks (splits * rows <= 8),
- *     unroll = 1 KiB loads in flight per wavefront (1|2|4).
+ *   W4A16_KERNEL_GENERIC: the scalar kernel, whatever the other arguments,
+ *     except where they name a shape of its matrix-core form: max_blocks = 1,
+ *     splits = wavefronts splitting K (1|2|4|8), rows = wavefronts on 8-row
+ *     blocks (splits * rows <= 8), unroll = 1 KiB loads in flight per
+ *     wavefront (1|2|4), on a layer it takes: group_size 32 or 64, M <= 8, K a
+ *     multiple of 128 up to 65536, activations and weights 16-byte and scales
+ *     256 / group_size-byte aligned, packed weights below 4 GiB.
  * The VALU and MFMA families need group_size 128, M <= 8 (16 for
  * W4A16_KERNEL_MFMA_ONESHOT, 2..16 for W4A16_KERNEL_MFMA_PAIR) and 16-byte
  * aligned activations and weights. workspace / workspace_bytes: as for

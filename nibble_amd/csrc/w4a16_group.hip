@@ -268,6 +268,12 @@ bool group_fits(int64_t M, int64_t N, int64_t K, int64_t G, const void* scales) 
     return N * (K / 2) < ((int64_t)1 << 32) && group_lds_bytes(1, K, 8) <= kLds;
 }
 
+// Whether (wavefronts on K, wavefronts on blocks, loads in flight) is a shape gemv_group is built for.
+bool group_shape(int sk, int sn, int depth) {
+    const auto of = [](int v, int top) { return v >= 1 && v <= top && (v & (v - 1)) == 0; };
+    return of(sk, 8) && of(depth, 4) && sn >= 1 && sn <= 8 && sk * sn <= 8;
+}
+
 // Launch shape, from a sweep of (SK, SN, D) over 16 layers (graph timing,
 // rotated weights; us of the shape taken against the next kind). M = 1: the
 // staged row is small, so one 8-row block a workgroup, 8 wavefronts on K (4096
@@ -291,8 +297,9 @@ void group_plan(int64_t M, int64_t N, int64_t K, int* sk, int* sn, int* depth) {
 int launch_group(int G, int sk, int sn, int depth, int M, const void* x, const uint8_t* w, const void* s, void* o,
                  int N, int K, hipStream_t stream) {
     using namespace w4a16;
-    if (!group_fits(M, N, K, G, s) || sk < 1 || sn < 1 || sk * sn > 8) {
-        set_last_error("group kernel: group size 32 or 64, M <= 8, K a multiple of 128, at most 8 wavefronts");
+    if (!group_fits(M, N, K, G, s) || !group_shape(sk, sn, depth)) {
+        set_last_error("group kernel: group size 32 or 64, M <= 8, K a multiple of 128, splits 1, 2, 4 or 8, unroll 1, 2 "
+                       "or 4, at most 8 wavefronts");
         return W4A16_ERR_CONFIG;
     }
     // rows past what LDS holds go in further launches of about equal size (the weights are read again)
@@ -303,10 +310,6 @@ int launch_group(int G, int sk, int sn, int depth, int M, const void* x, const u
         const int rows = (M - m0 + parts - i - 1) / (parts - i);
         const GroupKern kern = G == 32 ? (rows == 1 ? pick_group<32, 1>(sk, depth) : pick_group<32, 4>(sk, depth))
                                        : (rows == 1 ? pick_group<64, 1>(sk, depth) : pick_group<64, 4>(sk, depth));
-        if (kern == nullptr) {
-            set_last_error("group kernel: splits must be 1, 2, 4 or 8 and unroll 1, 2 or 4");
-            return W4A16_ERR_CONFIG;
-        }
         const int lds = (int)group_lds_bytes(rows, K, sk * sn);
         const int rc = ensure_lds(reinterpret_cast<const void*>(kern), lds);
         if (rc != W4A16_OK) return rc;

@@ -82,6 +82,7 @@ int launch_gemm3(int mt, int rb, int sn, int sk, bool paired, int M, const void*
                  void* o, int N, int K, hipStream_t stream);
 // w4a16_group.hip: group sizes 32 and 64 at M = 1..8
 bool group_fits(int64_t M, int64_t N, int64_t K, int64_t G, const void* scales);
+bool group_shape(int sk, int sn, int depth);
 void group_plan(int64_t M, int64_t N, int64_t K, int* sk, int* sn, int* depth);
 int launch_group(int G, int sk, int sn, int depth, int M, const void* x, const uint8_t* w, const void* s, void* o,
                  int N, int K, hipStream_t stream);
@@ -1400,7 +1401,9 @@ int run_plan(const Plan& p, const void* act, const uint8_t* packed, const void* 
             return w4a16_internal::launch_gemm3(p.rows, p.max_blocks, p.unroll, p.splits, false, (int)M, x, packed, s, o,
                                                 (int)N, (int)K, st);
         case W4A16_KERNEL_GENERIC:
-            if (p.max_blocks == 1 && aligned16(x) && aligned16(packed) && w4a16_internal::group_fits(M, N, K, G, s))
+            // anything but a shape of the matrix-core form on operands it takes is the scalar kernel, which needs no shape
+            if (p.max_blocks == 1 && w4a16_internal::group_shape(p.splits, p.rows, p.unroll) && aligned16(x) &&
+                aligned16(packed) && w4a16_internal::group_fits(M, N, K, G, s))
                 return w4a16_internal::launch_group((int)G, p.splits, p.rows, p.unroll, (int)M, x, packed, s, o, (int)N,
                                                     (int)K, st);
             return launch_generic((int)M, x, packed, s, o, (int)N, (int)K, (int)G, st);

@@ -48,6 +48,23 @@ def test_group_launch_shapes(gpu, m, group, splits, rows, depth):
     assert_parity(out, expected(x, p, s, group), f"M={m} G={group} {splits}x{rows} D={depth}")
 
 
+@pytest.mark.parametrize("rows,splits,depth", [(1, 3, 1), (0, 0, 0), (-1, 1, 1), (2, 8, 1), (9, 1, 1), (1, 16, 1),
+                                               (1, 2, 3), (1, 1, 8)])
+def test_generic_takes_any_other_arguments(gpu, rows, splits, depth):
+    """Arguments that are no shape of the matrix-core form are ignored: the scalar kernel's bits."""
+    x, p, s = make_case(2, 384, 24, seed=7, group_size=64)
+    xd, pd, sd = _on(gpu, x, p, s)
+    got = []
+    for max_blocks in (0, 1):
+        out = torch.full((2, 24), float("nan"), dtype=torch.float16, device=gpu)
+        print(f"[case] rows={rows} splits={splits} depth={depth} max_blocks={max_blocks}", flush=True)
+        _lib.linear_f16_tuned(xd, pd, sd, out, 64, _lib.KERNEL_GENERIC, rows, splits, depth, max_blocks)
+        torch.cuda.synchronize()
+        got.append(out)
+    assert_parity(got[0], expected(x, p, s, 64), "scalar")
+    assert torch.equal(*got)
+
+
 def test_group_scales_of_other_alignment_and_inf(gpu):
     """Scales that are only 2-byte aligned keep the scalar kernel; a non-finite
     scale or activation of one group reaches only its own outputs."""
