@@ -464,6 +464,24 @@ __device__ __forceinline__ void xcd_tile(int b, int nblocks, int& nbk, int& mbk)
     mbk = t - nbk * mblocks;
 }
 
+// Steps between the scheduling boundaries of gemm3_w4a16 (0: none). The
+// compiler fits a region's scheduling groups together in a time that grows
+// much faster than their number: with none, the four unrolled rounds of the
+// main loop are one region, and w4a16_gemm.hip took 11 minutes to compile (50
+// seconds now; the two shapes without a short region take half of that). A
+// boundary changes the register allocation as well, so each shape has the
+// region that ran best of 1, 4, 8, 16 steps and none (mean time against none
+// over M = 64..1024 of seven layers): (2, 2, 4, 1) 0.972; (4, 2, 4, 1) 0.957,
+// (4, 1, 4, 1) 1.000 and the SiLU form of (2, 2, 4, 1) 0.987; (2, 1, 2, 4)
+// 0.995; (2, 1, 1, 4) 0.985, the SiLU form of (2, 2, 1, 4) 0.993, (4, 1, 2, 2)
+// 1.02; (2, 1, 4, 2) 1.022 at best with boundaries.
+constexpr int gemm3_region(int mt, int rb, int sn, int sk, bool paired) {
+    if (mt == 2 && rb == 2 && sn == 4 && !paired) return 1;
+    if (sk == 1 || (mt == 2 && rb == 2 && sn == 2)) return 4;
+    if (mt == 2 && sn == 2) return 8;
+    return mt == 2 && sn == 4 ? 0 : 16;
+}
+
 template <int MT, int RB, int SN, int SK, bool PAIRED = false, int LA = 2>
 __global__ void __launch_bounds__(64 * SN * SK)
 gemm3_w4a16(const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16* __restrict__ scales,
@@ -620,6 +638,7 @@ gemm3_w4a16(const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16*
     decode(bt, 0, 0);
     constexpr int NM = MT * RB;              // MFMAs per step
     constexpr int PUTS = (UPT + 4) / 5;      // units put per step, steps 1..5
+    constexpr int REGION = gemm3_region(MT, RB, SN, SK, PAIRED);
     // round r = r0 + d on ring slot d; refill: request the rounds ahead (the last rounds of a row need none)
     auto round = [&](int d, int r, bool refill) __attribute__((always_inline)) {
         const int buf = d & 1;
@@ -668,6 +687,8 @@ gemm3_w4a16(const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16*
             for (int t = 0; t < MT; ++t) af[t] = an[t];
 #pragma unroll
             for (int rr = 0; rr < RB; ++rr) bt[rr] = bn[rr];
+            if constexpr (REGION > 0)
+                if ((8 * d + st) % REGION == REGION - 1) __builtin_amdgcn_sched_barrier(0);
         }
     };
     int r0 = 0;
