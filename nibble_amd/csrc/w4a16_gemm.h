@@ -482,8 +482,18 @@ constexpr int gemm3_region(int mt, int rb, int sn, int sk, bool paired) {
     return mt == 2 && sn == 4 ? 0 : 16;
 }
 
+// Wavefronts per SIMD that a shape's registers must leave room for: its own
+// workgroup's, and for (2, 2, 2, 2), whose grids run to 264 workgroups of 4
+// wavefronts on 256 CUs, those of a second one. At 206 + 64 registers it had
+// one resident, and the last 8 workgroups ran a round of their own: 2048 x 2 x
+// 5632 with SiLU at 144 and 192 rows 29.4 and 31.8 us against 26.8 and 28.5;
+// the bound costs it two spilled registers.
+constexpr int gemm3_waves(int mt, int rb, int sn, int sk) {
+    return mt == 2 && rb == 2 && sn == 2 && sk == 2 ? 2 : (sn * sk + 3) / 4;
+}
+
 template <int MT, int RB, int SN, int SK, bool PAIRED = false, int LA = 2>
-__global__ void __launch_bounds__(64 * SN * SK)
+__global__ void __launch_bounds__(64 * SN * SK, gemm3_waves(MT, RB, SN, SK))
 gemm3_w4a16(const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16* __restrict__ scales,
             f16* __restrict__ out, int M, int N, int K, int nblocks) {
     static_assert(!PAIRED || RB % 2 == 0, "paired tiles come in gate / up pairs");

@@ -728,3 +728,48 @@ def test_module_traces_whole(rows):
     assert len(graphs) == 1
     assert any("w4a16.linear" in target for target in graphs[0]) == (rows <= 512)
     assert any("w4a16.dequantize" in target for target in graphs[0]) == (rows > 512)
+
+
+def _built_kernels():
+    """name -> metadata of every kernel in the library as built (the code objects' own notes)."""
+    import struct
+
+    msgpack = pytest.importorskip("msgpack")
+    with open(_lib.LIB_PATH, "rb") as f:
+        blob = f.read()
+    kernels = {}
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    bundle = blob.find(magic)
+    while bundle >= 0:
+        entry = bundle + 32
+        for _ in range(struct.unpack_from("<Q", blob, bundle + 24)[0]):
+            offset, size, length = struct.unpack_from("<QQQ", blob, entry)
+            entry += 24 + length
+            if size:
+                kernels.update(_elf_kernels(blob[bundle + offset:bundle + offset + size], struct, msgpack))
+        bundle = blob.find(magic, bundle + 1)
+    return kernels
+
+
+def _elf_kernels(elf, struct, msgpack):
+    table, = struct.unpack_from("<Q", elf, 40)
+    size, count = struct.unpack_from("<HH", elf, 58)
+    for i in range(count):
+        kind, = struct.unpack_from("<I", elf, table + i * size + 4)
+        start, = struct.unpack_from("<Q", elf, table + i * size + 24)
+        if kind == 7 and elf[start + 12:start + 18] == b"AMDGPU":   # a note of this owner
+            _, text, _ = struct.unpack_from("<III", elf, start)
+            return {k[".name"]: k for k in msgpack.unpackb(elf[start + 20:start + 20 + text])["amdhsa.kernels"]}
+    return {}
+
+
+def test_gemm_shapes_that_count_on_two_workgroups_a_cu():
+    """(2, 2, 2, 2) of the 32x32 GEMM and its SiLU form, 4 wavefronts a
+    workgroup: registers (512 a lane of each SIMD, in blocks of 8) and LDS for
+    two workgroups on a CU, which a grid of 257..512 needs to run in one round."""
+    shapes = [k for name, k in _built_kernels().items() if "gemm3_w4a16ILi2ELi2ELi2ELi2E" in name]
+    assert len(shapes) == 2
+    for k in shapes:
+        assert k[".max_flat_workgroup_size"] == 256
+        assert -(-k[".vgpr_count"] // 8) * 8 * 2 <= 512, k
+    assert 2 * (2 * 2 * 64 * 136 * 2) <= 160 * 1024   # two staging buffers of 2 groups x 64 rows of 136 halves
