@@ -587,7 +587,14 @@ bool plan_prompt(int64_t M, int64_t N, int64_t K, Plan* p) {
         p->max_blocks = c.rb;
         p->splits = c.sk;
     }
+    // Up to 28 rows more than half of a 64-row tile is padding, of which the
+    // 16x16 kernel only re-reads the last row: it keeps those rows except on
+    // wide layers, where one round of the larger tiles does (us at M = 17 / 24:
+    // K x N 28672 x 8192 57.3 / 66.3 against 69.9 / 70.3, 1024 x 28672 9.7 /
+    // 10.4 against 10.8 / 10.9; but 14336 x 28672 0.84 / 0.76 of its time)
+    const bool few = M <= 28 && (N <= 16384 || K < 2048);
     for (const auto& c : k32) {
+        if (few) break;
         const double t = gemm_cost(c, 32, M, N, K);
         if (t >= best || !w4a16_internal::gemm3_instantiated(c.mt, c.rb, c.sn, c.sk, false)) continue;
         best = t;

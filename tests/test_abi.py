@@ -730,6 +730,32 @@ def test_module_traces_whole(rows):
     assert any("w4a16.dequantize" in target for target in graphs[0]) == (rows > 512)
 
 
+@pytest.mark.parametrize("m,k,n,kernel,rows,blocks,unroll,splits", [
+    (17, 28672, 8192, "gemm", 2, 2, 0, 4), (28, 28672, 6144, "gemm", 2, 2, 0, 4),      # more padding than rows
+    (29, 28672, 8192, "gemm32", 2, 1, 1, 4),
+    (17, 1024, 20480, "gemm", 2, 4, 0, 4), (28, 1024, 28672, "gemm", 2, 4, 0, 4),
+    (29, 1024, 28672, "gemm32", 2, 1, 4, 2),
+    (17, 8192, 28672, "gemm32", 2, 1, 4, 2), (17, 2048, 20480, "gemm32", 2, 1, 4, 2),   # wide layers
+    (24, 2048, 5632, "gemm", 2, 2, 0, 4), (17, 4096, 4096, "gemm", 1, 2, 0, 4),
+    (200, 5632, 2048, "gemm32", 2, 1, 1, 4), (384, 14336, 4096, "gemm32", 2, 1, 4, 2),
+    (700, 4096, 14336, "gemm32", 4, 1, 4, 1), (700, 2048, 5632, "gemm32", 2, 2, 4, 1),
+    (2048, 4096, 14336, "gemm32", 4, 2, 4, 1)])
+def test_prompt_plans(m, k, n, kernel, rows, blocks, unroll, splits):
+    """The shapes of least estimated time, which the torch op takes for M > 16."""
+    plan = _lib.plan_linear(ALIGNED, ALIGNED, m, n, k, 128, workspace=True)
+    assert plan == {"kernel": kernel, "rows": rows, "splits": splits, "unroll": unroll, "max_blocks": blocks}
+    assert _lib.linear_workspace_bytes(m, n, k) == 0
+
+
+@pytest.mark.parametrize("m,k", [(16, 4096), (9, 2048), (17, 896), (64, 128), (200, 896)])
+def test_prompt_plans_outside_the_estimate(m, k):
+    """Up to 16 rows, and rows shorter than 1024 weights, plan as without a workspace where none is used."""
+    for n in (520, 4096, 20480):
+        if _lib.linear_workspace_bytes(m, n, k) == 0:
+            plain = _lib.plan_linear(ALIGNED, ALIGNED, m, n, k, 128)
+            assert _lib.plan_linear(ALIGNED, ALIGNED, m, n, k, 128, workspace=True) == plain
+
+
 def _built_kernels():
     """name -> metadata of every kernel in the library as built (the code objects' own notes)."""
     import struct
