@@ -49,21 +49,22 @@ NATIVE_GEMM_MAX_ROWS = 512
 def gemm_max_rows(n: int, k: int) -> int:
     """Rows up to which the W4A16 GEMM of a layer keeps up with dequantize + the
     dense GEMM: a sweep of 513..1024 rows over layers of up to 24M weights
-    (graph timing, rotated weights), in which it loses no more than 1.5%
+    (graph timing, rotated weights), in which it loses no more than 1%
     anywhere below these lines. Its tiles fill whole rounds of the 256 CUs on
-    small and narrow layers (K x N at 1024 rows, us: 5632 x 2048 36.6 against
-    45.3, 14336 x 1024 57.7 against 61.9, 2048 x 4096 26.6 against 34.8).
-    Others start a second round past 704 rows (4096 x 5632 at 704 50.6 against
-    54.0, at 705 62.8 against 55.0; 1408 x 16384 at 704 45.6 against 50.5, at
-    1024 64.9 against 58.2), the widest at once (1024 x 20480 at 576 49.1
-    against 43.5). Rows shorter than 1024 weights run shapes chosen by their
-    grid alone, which lose here and there past 512 outputs (128 x 1024 at 576
-    12.1 against 8.2)."""
-    if n * k > 24_000_000 or (k < 1024 and n > 512):
+    small and narrow layers (K x N at 1024 rows, us: 5632 x 2048 35.2 against
+    44.4, 14336 x 1024 55.3 against 60.8, 2048 x 4096 25.9 against 34.4).
+    Others start a further round past 704 rows (4096 x 5632 at 704 46.6
+    against 54.1, at 705 59.1 against 54.9; 1408 x 16384 at 704 43.2 against
+    49.5, at 960 57.9 against 55.6), the widest at once (1024 x 20480 at 576
+    44.7 against 43.0). Rows shorter than 1024 weights run shapes chosen by
+    their grid alone, which lose here and there past 512 outputs (128 x 1024
+    at 576 12.0 against 8.3)."""
+    weights = n * k
+    if weights > 24_000_000 or (k < 1024 and n > 512):
         return NATIVE_GEMM_MAX_ROWS
-    if n <= 2048 or n * k <= (12_000_000 if n <= 4096 else 9_000_000):
+    if n <= 2048 or weights <= 12_000_000 or (n <= 4096 and weights <= 17_500_000):
         return 2 * NATIVE_GEMM_MAX_ROWS
-    return 704 if n <= 5632 or (n <= 16384 and k <= 2048) else NATIVE_GEMM_MAX_ROWS
+    return 704 if n <= 16384 else NATIVE_GEMM_MAX_ROWS
 
 
 class QuantizedLinear(torch.nn.Module):

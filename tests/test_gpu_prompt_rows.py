@@ -51,10 +51,10 @@ def test_rows_that_take_the_gemm():
 
 @pytest.mark.parametrize("k,n,rows", [
     (2048, 2048, 1024), (5632, 2048, 1024), (11008, 2048, 1024), (14336, 1536, 1024), (2048, 4096, 1024),
-    (1024, 8192, 1024), (128, 512, 1024),                                         # faster up to 1024 rows
-    (4096, 2560, 1024), (5632, 2560, 704), (8192, 2560, 704), (4096, 4096, 704), (2048, 5632, 704),
-    (4096, 5632, 704), (2048, 11264, 704), (1408, 16384, 704), (1024, 16384, 704),   # slower past 704
-    (1024, 20480, 512), (2816, 8192, 512), (128, 1024, 512), (512, 16384, 512), (4096, 6144, 512)])
+    (4096, 4096, 1024), (2048, 5632, 1024), (1024, 8192, 1024), (128, 512, 1024),    # faster up to 1024 rows
+    (8192, 2560, 704), (4096, 5632, 704), (2048, 11264, 704), (1408, 16384, 704), (1024, 16384, 704),
+    (2816, 8192, 704),                                                               # slower past 704
+    (1024, 20480, 512), (128, 1024, 512), (512, 16384, 512), (4096, 6144, 512)])
 def test_rows_up_to_which_the_gemm_keeps_up(k, n, rows):
     assert gemm_max_rows(n, k) == rows
 
