@@ -552,11 +552,12 @@ bool plan_gemm32_silu(int64_t M, int64_t inter, int64_t K, Plan* out) {
 // tiles; past that a further round, of which a shape that fits twice on a CU
 // hides the part of `hide` that its last round leaves empty. a, b and hide
 // from a sweep of every shape over M 24..1024 on eight layers (graph timing,
-// rotated weights), which this picks the fastest of, or one within 6%, in all
-// of 64 cases. Where the fixed thresholds above lose: M = 384, 14336 x
-// 4096 77 against 135 us; M = 200 56 against 70; M = 384, 5632 x 2048 23.4
-// against 31.5; M = 700, 2048 x 5632 26 against 35; M = 700, 4096 x 14336 110
-// against 126.
+// rotated weights). Against the fixed thresholds above, over 1800 random
+// layers (K 1024..14336, N 512..16384) at 17..512 rows: 0.82 of their time in
+// the mean, at most 1.15, more than 1.04 on 12 (small grids, where a 16x16
+// shape is faster than a K + b). M = 384, 14336 x 4096 77 against 135 us; M =
+// 200 56 against 70; M = 384, 5632 x 2048 23.4 against 31.5; M = 700, 2048 x
+// 5632 26 against 35; M = 700, 4096 x 14336 110 against 126.
 struct GemmCost {
     int mt, rb, sn, sk;
     double a, b, hide;
@@ -564,7 +565,12 @@ struct GemmCost {
 
 double gemm_cost(const GemmCost& c, int tile, int64_t M, int64_t N, int64_t K) {
     const int64_t rows = (int64_t)tile * c.mt, cols = (int64_t)tile * c.rb * c.sn;
-    const int64_t tiles = ((N + cols - 1) / cols) * ((M + rows - 1) / rows);
+    int64_t blocks = (N + cols - 1) / cols;
+    // the 16x16 kernel's XCDs take whole weight blocks, and the one with the
+    // most decides (6144 x 832 at 597 rows: 13 blocks of 19 tiles, 38 of them
+    // on the 32 CUs of five XCDs, 47 us for an estimate of 25)
+    if (tile == 16) blocks = (blocks + 7) & ~(int64_t)7;
+    const int64_t tiles = blocks * ((M + rows - 1) / rows);
     const double rounds = (double)((tiles + 255) / 256), last = (double)((tiles - 1) % 256 + 1) / 256.0;
     return (rounds - (rounds > 1 ? c.hide * (1.0 - last) : 0.0)) * (c.a * (double)K / 1024.0 + c.b);
 }

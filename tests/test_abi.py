@@ -737,6 +737,8 @@ def test_module_traces_whole(rows):
     (29, 1024, 28672, "gemm32", 2, 1, 4, 2),
     (17, 8192, 28672, "gemm32", 2, 1, 4, 2), (17, 2048, 20480, "gemm32", 2, 1, 4, 2),   # wide layers
     (24, 2048, 5632, "gemm", 2, 2, 0, 4), (17, 4096, 4096, "gemm", 1, 2, 0, 4),
+    (597, 6144, 832, "gemm32", 2, 1, 2, 4), (324, 8960, 768, "gemm32", 2, 1, 1, 4),   # 13 and 12 blocks of 64 on 8 XCDs
+    (44, 3328, 2688, "gemm", 2, 2, 0, 4), (45, 2048, 1344, "gemm", 1, 2, 0, 4),
     (200, 5632, 2048, "gemm32", 2, 1, 1, 4), (384, 14336, 4096, "gemm32", 2, 1, 4, 2),
     (700, 4096, 14336, "gemm32", 4, 1, 4, 1), (700, 2048, 5632, "gemm32", 2, 2, 4, 1),
     (2048, 4096, 14336, "gemm32", 4, 2, 4, 1)])
