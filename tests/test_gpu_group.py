@@ -86,3 +86,40 @@ def test_group_scales_of_other_alignment_and_inf(gpu):
         assert torch.equal(finite, torch.isfinite(got[0]))
         assert finite[0].sum() == 23 and not finite[0, 3]
         assert torch.allclose(got[0][finite], got[1][finite], rtol=1e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("group", [32, 64])
+@pytest.mark.parametrize("m,k,splits", [(1, 128, 0), (1, 1152, 0), (4, 640, 0), (8, 384, 0), (8, 2176, 8), (3, 1152, 1)])
+def test_group_infinite_scales(gpu, m, k, group, splits):
+    """An infinite scale gives what the sum over code * scale * x gives: NaN
+    with a code or an activation of 0 in its group or products of both signs,
+    else an infinity of their sign; other rows of the layer keep their bits."""
+    n, groups = 12, k // group
+    x, p, s = make_case(m, k, n, seed=k + m + group, group_size=group)
+    plain = s.clone()
+    x[0] = 1.0 + x[0].abs()                       # one sign in activation row 0
+    inf = float("inf")
+    s[0, groups // 2] = inf                       # random codes: both signs
+    s[1, 0], p[1, :group // 2] = inf, 0x33        # one sign
+    s[2, groups - 1], p[2, -group // 2:] = -inf, 0x33
+    s[3, 0], p[3, :group // 2], p[3, 0] = inf, 0x33, 0x03   # one code of 0
+    s[4, 0], s[4, groups - 1] = inf, -inf         # one sign each, of different signs
+    p[4, :group // 2], p[4, -group // 2:] = 0x33, 0x33
+    s[5, groups // 2] = float("nan")
+    xd, pd, sd = _on(gpu, x, p, s)
+    out = torch.full((m, n), float("nan"), dtype=torch.float16, device=gpu)
+    print(f"[case] infinite scales M={m} K={k} G={group} splits={splits}", flush=True)
+    if splits:
+        _lib.linear_f16_tuned(xd, pd, sd, out, group, _lib.KERNEL_GENERIC, 1, splits, 2, 1)
+    else:
+        _lib.linear_f16(xd, pd, sd, out, group)
+    torch.cuda.synchronize()
+    got = out.float().cpu()
+    codes = ((torch.stack((p & 15, p >> 4), dim=-1).reshape(n, k).int() ^ 8) - 8).float()
+    wide = codes * s.float().repeat_interleave(group, dim=1)
+    terms = x.float().unsqueeze(1) * wide.unsqueeze(0)           # [m, n, k]
+    want = terms.sum(dim=2)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isneginf(), want.isneginf())
+    assert got[0, 0].isnan() and got[0, 1] == inf and got[0, 2] == -inf and got[0, 3:6].isnan().all()
+    assert_parity(out[:, 6:], expected(x, p[6:], plain[6:], group), f"M={m} K={k} G={group}")
