@@ -99,12 +99,14 @@ int64_t w4a16_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t gr
  * M = 12..16 layers of K = 5632 (N <= 4096), 8192 or 14336 (N <= 8192) and
  * M = 3..8 layers of K = 28672 (N = 4096..8192) and M = 5..8 layers of
  * K = 8192 with N >= 16384 the paired ring kernel over K slices; the fp32
- * partial sums are added in slice
- * order by a second launch; M > 16 takes the GEMM shape of the least estimated
- * time (no workspace bytes used). workspace == NULL routes exactly as w4a16_linear_f16;
- * a smaller non-NULL workspace is W4A16_ERR_CONFIG. The torch op
- * w4a16::linear (reference csrc/int4_linear.cpp:16-28) calls this entry
- * point with a workspace from the caching allocator.
+ * partial sums are added in slice order by a second launch; M > 16 takes the
+ * GEMM shape of the least estimated time and uses no workspace bytes (callers
+ * with none to give get that route from w4a16_linear_noalloc_f16, which
+ * touches no scratch at M > 16). workspace == NULL routes exactly as
+ * w4a16_linear_f16; a smaller non-NULL workspace is W4A16_ERR_CONFIG. The
+ * torch op w4a16::linear (reference csrc/int4_linear.cpp:16-28) calls this
+ * entry point up to M = 16, with a workspace from the caching allocator, and
+ * w4a16_linear_noalloc_f16 above.
  */
 int w4a16_linear_ws_f16(const void* activations, const uint8_t* packed_weights,
                         const void* scales, void* output, int64_t M, int64_t N,

@@ -1,8 +1,9 @@
 // Thin libtorch shim over the W4A16 C ABI: registers the torch ops
 // w4a16::linear and w4a16::dequantize with the schemas of reference
-// csrc/int4_linear.cpp:16-23 and w4a16::quantize (the reference quantizes in torch ops), implemented on the CUDA dispatch key (which is
-// the HIP device on PyTorch-ROCm), and exposes an empty Python module so that
-// importing the extension registers the ops (reference csrc/int4_linear.cpp:30).
+// csrc/int4_linear.cpp:16-23 and w4a16::quantize (the reference quantizes in
+// torch ops), implemented on the CUDA dispatch key (which is the HIP device on
+// PyTorch-ROCm), and exposes an empty Python module so that importing the
+// extension registers the ops (reference csrc/int4_linear.cpp:30).
 //
 // Tensor-level checks use the reference's messages (reference
 // csrc/int4_linear_kernel.cu:646-691, :809-841); shape relations and launches
@@ -52,15 +53,21 @@ at::Tensor linear(const at::Tensor& activations, const at::Tensor& packed_weight
     at::Tensor output = at::empty({M, N}, activations.options());
     if (M * N == 0) return output;
 
+    void* const stream = current_stream(activations.device());
+    if (M > 16) {   // prompt rows: no form of theirs has partial sums, so nothing of the library's scratch is used
+        rc = w4a16_linear_noalloc_f16(activations.data_ptr(), packed_weights.data_ptr<uint8_t>(), scales.data_ptr(),
+                                      output.data_ptr(), M, N, K, group_size, stream);
+        TORCH_CHECK(rc == W4A16_OK, w4a16_last_error());
+        return output;
+    }
     // partial sums of the split-K kernel, from the caching allocator (so the
-    // op stays graph-capture safe). Prompt rows need none, and any pointer
-    // leaves their GEMM's shape to the library
+    // op stays graph-capture safe)
     const int64_t ws_bytes = w4a16_linear_workspace_bytes(M, N, K, group_size);
     at::Tensor workspace;
     if (ws_bytes > 0) workspace = at::empty({(ws_bytes + 3) / 4}, activations.options().dtype(at::kFloat));
     rc = w4a16_linear_ws_f16(activations.data_ptr(), packed_weights.data_ptr<uint8_t>(), scales.data_ptr(),
-                             output.data_ptr(), M, N, K, group_size,
-                             ws_bytes > 0 ? workspace.data_ptr() : M > 16 ? output.data_ptr() : nullptr, ws_bytes, current_stream(activations.device()));
+                             output.data_ptr(), M, N, K, group_size, ws_bytes > 0 ? workspace.data_ptr() : nullptr,
+                             ws_bytes, stream);
     TORCH_CHECK(rc == W4A16_OK, w4a16_last_error());
     return output;
 }
