@@ -229,16 +229,18 @@ def test_decode_attention_split_long_caches(gpu, heads, kv, pos, S, splits):
     assert torch.allclose(kd[:, pos].cpu().float(), k_new.float(), rtol=2 ** -10, atol=2 ** -14)
 
 
-def test_decode_attention_split_out_of_range_and_rejects(gpu):
-    S, heads, kv = 256, 8, 2
+@pytest.mark.parametrize("S", [256, 1024, 1025, 1100])   # one launch up to 1024 slots, the split and merge launches past it
+def test_decode_attention_split_out_of_range_and_rejects(gpu, S):
+    heads, kv = 8, 2
     qkv = torch.randn(((heads + 2 * kv) * 64,)).to(torch.float16).to(gpu)
     kd = torch.zeros((kv, S, 64), dtype=torch.float16, device=gpu)
     vd = torch.zeros_like(kd)
     cos, sin = _tables(S)
     cos, sin = cos.to(gpu), sin.to(gpu)
     out = torch.zeros((heads * 64,), dtype=torch.float16, device=gpu)
-    ws = torch.zeros((heads * 4 * 66,), dtype=torch.float32, device=gpu)
+    ws = torch.zeros((heads * 4 * 66,), dtype=torch.float32, device=gpu)   # what an invalid position leaves unwritten
     for bad in (S, -1):
+        out.zero_()
         position = torch.tensor([bad], dtype=torch.int64, device=gpu)
         _lib.decode_attention_split_f16(qkv, kd, vd, cos, sin, position, out, heads, kv, 4, ws)
         torch.cuda.synchronize()
@@ -865,18 +867,20 @@ def test_attention_o_step_matches_two_launch_step(gpu):
     assert torch.allclose(model.k_cache[:, :, p].float(), ref_k[:, :, p].float(), rtol=1e-2, atol=1e-2)
 
 
-def test_split_attention_step(gpu):
-    """A 640-slot cache takes the split decode attention (5 shares per head):
-    from the same state after a 600-token prompt, the fused step against the
+@pytest.mark.parametrize("slots,tokens,shares", [(640, 600, 5), (1152, 1100, 9)])
+def test_split_attention_step(gpu, slots, tokens, shares):
+    """Caches past 512 slots call the split decode attention, which runs one
+    workgroup per head on 640 slots and 9 shares per head with a merge launch
+    on 1152: from the same state after a prompt, the fused step against the
     torch-op step and against the fused step with one workgroup per head
     (logits |err| <= 2e-2 (1 + |ref|)); graphed tokens equal eager ones."""
     from dataclasses import replace
 
     from nibble_amd.llama import LlamaDecoder
 
-    model = LlamaDecoder(replace(_small_cfg(), max_seq_len=640), device=gpu, seed=5)
-    assert model.attn_splits == 5
-    prompt = torch.randint(0, 512, (600,), generator=torch.Generator().manual_seed(6)).to(gpu)
+    model = LlamaDecoder(replace(_small_cfg(), max_seq_len=slots), device=gpu, seed=5)
+    assert model.attn_splits == shares
+    prompt = torch.randint(0, 512, (tokens,), generator=torch.Generator().manual_seed(6)).to(gpu)
     model.prefill(prompt)
     state = (model.k_cache.clone(), model.v_cache.clone(), model.token.clone(), model.position.clone(),
              model.x_buf.clone())
@@ -890,13 +894,13 @@ def test_split_attention_step(gpu):
         torch.cuda.synchronize()
         return model.logits.float().cpu(), model.k_cache.clone()
 
-    ref, ref_k = step(False, 5)
-    got, got_k = step(True, 5)
+    ref, ref_k = step(False, shares)
+    got, got_k = step(True, shares)
     one, _ = step(True, 0)
     for other in (ref, one):
         assert torch.all((got - other).abs() <= 2e-2 * (1 + other.abs())), float((got - other).abs().max())
-    assert torch.allclose(got_k[:, :, 600].float(), ref_k[:, :, 600].float(), rtol=1e-2, atol=1e-2)
-    model.attn_splits = 5
+    assert torch.allclose(got_k[:, :, tokens].float(), ref_k[:, :, tokens].float(), rtol=1e-2, atol=1e-2)
+    model.attn_splits = shares
     eager = model.generate(prompt, 6, use_graph=False)
     model.prefill(prompt)
     model.capture()

@@ -810,3 +810,24 @@ def test_dequantize_small_and_ragged(gpu, group, n, groups):
     torch.cuda.synchronize()
     ref = torch.from_numpy(oracle.dequantize_f16(p.numpy(), s.numpy(), group))
     assert torch.equal(out.cpu().view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("n,k,group", [(65536, 2048, 128),   # 256 MiB of output: the last with plain stores
+                                       (65537, 2048, 128),   # the first with non-temporal ones
+                                       (69911, 1920, 96),    # a ragged last workgroup and a group that is no power of two
+                                       (1048577, 128, 32)])
+def test_dequantize_past_the_streaming_threshold(gpu, n, k, group):
+    """Outputs around 256 MiB, past which the stores are non-temporal: every
+    fp16 bit against the torch product of codes and scales."""
+    gen = torch.Generator(device=gpu).manual_seed(n)
+    p = torch.randint(0, 256, (n, k // 2), generator=gen, dtype=torch.uint8, device=gpu)
+    s = (torch.rand((n, k // group), generator=gen, device=gpu) * 4 - 2).to(torch.float16)
+    print(f"[case] dequantize N={n} K={k} G={group}", flush=True)
+    out = torch.ops.w4a16.dequantize(p, s, group)
+    torch.cuda.synchronize()
+    rows = (1 << 25) // k
+    for at in range(0, n, rows):
+        wide = p[at:at + rows].to(torch.int16)
+        codes = torch.stack((((wide & 15) ^ 8) - 8, ((wide >> 4) ^ 8) - 8), dim=-1).reshape(-1, k // group, group)
+        ref = (codes.float() * s[at:at + rows].float().unsqueeze(-1)).to(torch.float16).reshape(-1, k)
+        assert torch.equal(out[at:at + rows].view(torch.int16), ref.view(torch.int16)), at
