@@ -98,12 +98,15 @@ int w4a16_decode_attention_f16(const void* qkv, void* k_cache, void* v_cache,
 
 /*
  * w4a16_decode_attention_f16 with each head's slots 0 .. position split into
- * up to `splits` shares (share s: the 64-slot chunks s, s + splits, ..), one workgroup per head and share
- * (num_heads x splits workgroups, where the unsplit form has num_heads), then
- * a second launch that merges the shares' softmax states per head. workspace:
- * num_heads * splits * 66 fp32 (264 bytes per head and share, 4-byte
- * aligned), overwritten by every call; calls that share one must not run
- * concurrently. 1 <= splits <= 64; other arguments, output and NaN rows as
+ * `splits` shares (share s: the 64-slot chunks s, s + splits, ..), one
+ * workgroup per head and share (num_heads x splits workgroups, where the
+ * unsplit form has num_heads), then a second launch that merges the shares'
+ * softmax states per head. Caches of up to 1024 slots (max_seq_len) are not
+ * split: there one launch is faster at every position, and the call is
+ * w4a16_decode_attention_f16 after its own checks. workspace: num_heads *
+ * splits * 66 fp32 (264 bytes per head and share, 4-byte aligned), asked for
+ * on every call, overwritten by those that split; calls that share one must
+ * not run concurrently. 1 <= splits <= 64; other arguments, output and NaN rows as
  * w4a16_decode_attention_f16 (the new k / v rows are appended once).
  * Replaces (reference): the same attention as w4a16_decode_attention_f16.
  */

@@ -47,14 +47,14 @@ namespace w4a16 {
 //      sum_w l_w e^(m_w - M), rounded to fp16 (a wavefront with no chunk has
 //      l_w = 0 and drops out).
 // Slots past p get weight exactly 0. A position outside [0, S) writes NaN
-// to the head's output and touches no cache slot. Every load that does not
-// depend on the position (cache rows of each wavefront's first chunk, q, k,
-// v) is requested before the position arrives.
+// to the head's output and touches no cache slot. q, k, v and the cache rows
+// of each wavefront's first chunk are requested before the position arrives.
 // ---------------------------------------------------------------------------
 // SPLIT: workgroup (hq, s) of gridDim.y attends a share of the slots 0 .. p
 // (chunks s, s + gridDim.y, ..: which ones does not depend on the position,
-// so the first of each wavefront is requested before it arrives) and writes
-// its unnormalised state to partial[hq][s] = {max, sum, acc[64]} for
+// so the first one, wavefront 0's, is requested before it arrives; those of
+// wavefronts 1 .. lie further on, and are requested once the position says
+// that they hold slots) and writes its unnormalised state to partial[hq][s] = {max, sum, acc[64]} for
 // decode_attention_merge; only share 0 appends the new k / v rows.
 // Bound: a chain of latencies (launch, position, first rows, merge launch),
 // not bytes. Graph timing, 32 / 4 heads, against keys read a row per lane and
@@ -1638,8 +1638,10 @@ int w4a16_decode_attention_split_f16(const void* qkv, void* k_cache, void* v_cac
                     "split attention: caches 16-byte aligned, fp16 buffers 2-byte, workspace 4-byte aligned");
     // caches of up to 1024 slots: one workgroup per head is faster than two
     // launches at every position (32 / 4 heads, us: position 500 5.6 against
-    // 7.7, 1000 7.5 against 7.7); on longer ones it loses from about position
-    // 1400 on (2048 slots, position 2047: 11.1 against 9.0)
+    // 7.7, 1000 7.5 against 7.7; and over 8 combinations of 4 .. 128 heads,
+    // 640 and 1024 slots, 0.61 to 0.99 of the split form's time); on longer
+    // ones it loses from about position 1400 on (2048 slots, position 2047:
+    // 11.1 against 9.0), which the host does not know
     if (max_seq_len <= kSplitMinSlots)
         return w4a16_decode_attention_f16(qkv, k_cache, v_cache, cos_table, sin_table, position, output, num_heads,
                                           num_kv_heads, head_dim, max_seq_len, stream);

@@ -435,10 +435,11 @@ gemm2_w4a16(const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16*
 // k = 64 h + 8 s .. + 7, so a lane's weights of one group are bytes 32 h ..
 // 32 h + 31 of its row's 64-byte group (two 16-byte loads, word s % 4 of
 // the first or second) and its A fragment of step s is the 16 contiguous
-// bytes at halves 64 h + 8 s of its activation row's staged group. Decode,
-// staging (rows of 136 halves), the ring of weight rounds, the XCD-aware grid
-// and the fixed-order SK reduction are those of gemm2_w4a16, with tiles of
-// 32 rows.
+// bytes at halves 64 h + 8 s of its activation row's staged group. Decode, the
+// staged rows of 136 halves, the ring of weight rounds and the fixed-order SK
+// reduction are those of gemm2_w4a16, with tiles of 32 rows; the rounds are
+// software-pipelined (below) and the grid holds the tiles alone, which the
+// XCDs share evenly (xcd_tile).
 // ---------------------------------------------------------------------------
 __host__ __device__ constexpr int64_t gemm3_lds_bytes(int mt, int rb, int sn, int sk) {
     return (int64_t)2 * sk * 32 * mt * kGemmRow * 2 > (int64_t)(sk - 1) * sn * mt * rb * 64 * 64

@@ -318,7 +318,10 @@ bool group_shape(int sk, int sn, int depth) {
 // 6.8 against 7.9 for 8 x 1), 2 x 4 on wide layers of short rows (4096 x 14336
 // at M = 4 10.9 against 12.7), 8 x 1 on narrow ones (5632 x 2048 7.6 against
 // 8.5). One load in flight a wavefront is enough while other workgroups share
-// the CU; 2 where a wavefront has more than five pairs or stages many rows.
+// the CU; 2 where a wavefront has more than five pairs or stages many rows. 4
+// runs through the tuned entry point only: it loses on rows of up to 4096
+// weights (4096 x 4096, G = 64, M = 1: 6.7 against 5.1) and on most of 14336,
+// and would win on rows of 28672 (x 8192: 30.4 against 37.2).
 void group_plan(int64_t M, int64_t N, int64_t K, int* sk, int* sn, int* depth) {
     const int64_t pairs = (K / 128 + 1) / 2;
     int k = M == 1 ? (N >= 5120 ? 4 : 8) : N >= 8192 && K <= 4096 ? 2 : N >= 4096 ? 4 : 8;

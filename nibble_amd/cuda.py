@@ -84,8 +84,10 @@ def linear_cuda(
 ) -> torch.Tensor:
     """Fused W4A16 linear on the GPU (reference ``w4a16/cuda.py:52-69``).
 
-    group_size 128 with 16-byte aligned operands and M <= 8 runs the tuned
-    gfx950 kernels; anything else runs the generic HIP kernel.
+    group_size 128 with 16-byte aligned operands runs the tuned gfx950 kernels
+    (up to 16 rows) and the W4A16 GEMM (above); group sizes 32 and 64 at M <= 8
+    with K a multiple of 128 run their matrix-core kernel; anything else runs
+    the scalar HIP kernel.
     """
     _require_extension()
     # the overload itself: naming the packet looks it up on every call (about 1 us)

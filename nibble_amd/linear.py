@@ -8,8 +8,9 @@ Mirrors reference ``w4a16/linear.py`` (constructor checks, buffers
 * CPU tensors: the pure-PyTorch ``linear_reference``;
 * GPU tensors, ``fused`` and M <= ``FUSED_MAX_ROWS``: ``w4a16::linear``
   (the gfx950 GEMV / small-batch kernels);
-* GPU tensors, ``fused``, group_size 128 and M <= ``NATIVE_GEMM_MAX_ROWS``
-  (prompts): ``w4a16::linear`` as well, which runs the W4A16 MFMA GEMM (at
+* GPU tensors, ``fused``, group_size 128 and M <= ``native_max_rows``
+  (prompts; 512, 704 or 1024 rows by the layer's sizes, see
+  ``gemm_max_rows``): ``w4a16::linear`` as well, which runs the W4A16 MFMA GEMM (at
   9..16 rows of long rows, its 16-row paired form) on weights decoded in
   registers, bit-identical to the dequantized fp16 weights, with fp32
   accumulation; the reference sends these rows to dequantize + cuBLAS, and
@@ -35,14 +36,13 @@ from nibble_amd.reference import dequantize_weights, linear_reference
 
 # Largest M routed to the fused kernels; larger M dequantizes and uses a GEMM.
 FUSED_MAX_ROWS = 8
-# Largest M routed to the W4A16 GEMM when fused (group size 128): measured
-# against dequantize + hipBLASLt on the 1.1B / 8B / 70B layers (e.g. M = 256,
-# K 4096 x N 14336: 45 us against 81 us; M = 64, 5632 x 2048: 10 us against
-# 32 us; M = 512: 69 against 95 us, 14336 x 4096 86 against 117, 8192 x 28672
-# 264 against 331, and every other swept layer faster too); from M = 1024
-# dequantize + hipBLASLt wins on the wide layers (4096 x 14336 138 against
-# 131 us, 2048 x 11264 75 against 69) and on most layers at M = 2048, so
-# longer prompts keep it.
+# Largest M routed to the W4A16 GEMM when fused (group size 128) on any layer:
+# measured against dequantize + hipBLASLt on the 1.1B / 8B / 70B layers (K x N,
+# us: M = 256, 4096 x 14336 43.7 against 74.2; M = 64, 5632 x 2048 11.6 against
+# 26.7; M = 512, 4096 x 14336 72.7 against 84.2, 14336 x 4096 86.5 against
+# 109.0, 8192 x 28672 275 against 281, and every other swept layer faster too).
+# Wide layers lose from M = 1024 (4096 x 14336 141.8 against 117.7) and nearly
+# every one at M = 2048 (2048 x 11264 118.0 against 97.2).
 NATIVE_GEMM_MAX_ROWS = 512
 
 

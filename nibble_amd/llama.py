@@ -283,13 +283,13 @@ class LlamaDecoder(torch.nn.Module):
         self.x_buf = torch.zeros((h,), dtype=torch.float16, device=device)
         self.qkv_buf = torch.zeros((h + 2 * kv,), dtype=torch.float16, device=device)
         self.attn_buf = torch.zeros((cfg.num_heads * cfg.head_dim,), dtype=torch.float16, device=device)
-        # caches past 512 slots: the decode attention split into shares of the
-        # slots (a workgroup per head and share, 256 workgroups where the heads
-        # allow) and merged per head; 0 keeps one workgroup per head. 1.1B
-        # model, graph-replayed decode: 2048 slots at position 1500 1837
-        # against 1597 tok/s, 1024 at 900 1907 against 1830, 512 at 300 1970
-        # against 2030 (so 512 slots keep the single launch); at most 64
-        # shares, the split launch's limit
+        # caches past 512 slots: the split decode attention with these shares
+        # (256 workgroups where the heads allow, at most the launch's 64; 0
+        # keeps the plain entry point). It splits caches past 1024 slots, a
+        # workgroup per head and share and a merge per head: 1.1B model,
+        # graph-replayed decode, 2048 slots at position 1500 2061 against 1961
+        # tok/s; up to 1024 it runs one workgroup per head as well, and does
+        # not read the workspace
         self.attn_splits = (min(max(1, 256 // cfg.num_heads), max(1, cfg.max_seq_len // 128), 64)
                             if cfg.max_seq_len > 512 else 0)
         self.attn_ws = torch.empty((max(1, cfg.num_heads * self.attn_splits * 66),), dtype=torch.float32,
