@@ -62,18 +62,22 @@ def _require_extension() -> None:
         ) from _EXTENSION_LOAD_ERROR
 
 
-def addressable(tensor: torch.Tensor) -> bool:
-    """Whether a choice may look at where this tensor's memory starts: an
-    ordinary tensor of a call that runs now. False for a traced call (its
-    graph also serves other tensors), under a dispatch mode, for a wrapper of
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+_transformed = torch._C._functorch.is_functorch_wrapped_tensor
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+
+
+def addressable(*tensors: torch.Tensor) -> bool:
+    """Whether a choice may look at where these tensors' memory starts: ordinary
+    tensors of a call that runs now. False for a traced call (its graph also
+    serves other tensors), under a dispatch mode, for a wrapper of
     ``torch.func`` and for a subclass, which may have no memory of their own."""
-    return (
-        not torch.compiler.is_compiling()
-        and type(tensor) in (torch.Tensor, torch.nn.Parameter)
-        and not torch.jit.is_tracing()
-        and torch._C._len_torch_dispatch_stack() == 0
-        and not torch._C._functorch.is_functorch_wrapped_tensor(tensor)
-    )
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or _dispatch_modes():
+        return False
+    for tensor in tensors:
+        if type(tensor) not in _PLAIN or _transformed(tensor):
+            return False
+    return True
 
 
 def linear_cuda(

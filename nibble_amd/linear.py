@@ -161,7 +161,8 @@ class QuantizedLinear(torch.nn.Module):
         rows = flat.shape[0]
         if rows > self.native_max_rows or rows <= NATIVE_GEMM_MAX_ROWS:
             return rows <= self.native_max_rows
-        return all(addressable(t) and t.data_ptr() % 16 == 0 for t in (flat, self.packed_weights))
+        packed = self.packed_weights
+        return addressable(flat, packed) and (flat.data_ptr() | packed.data_ptr()) % 16 == 0
 
     def _dequant_linear(self, activations: torch.Tensor) -> torch.Tensor:
         """fp16 weight matrix from the packed codes, then a dense GEMM."""
